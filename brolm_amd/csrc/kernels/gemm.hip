@@ -16,8 +16,10 @@
 //    contiguous run of tiles that share weight columns in its own L2.
 //  - gemm_kernel<FMT> (other shapes): 64x64 block tile, K step 32, 4
 //    wavefronts each a 32x32 quadrant of 16x16x16 MFMAs.
+// Quantized weights with K a multiple of 256 and 16-byte aligned operands run
+// gemm_quant.hip instead, at any M above 16 (gemm_quant_ok).
 #include "carrier_layout.h"
-#include "common.h"
+#include "gemm_job.h"
 
 namespace bx {
 namespace {
@@ -295,32 +297,6 @@ __device__ __forceinline__ u4v decode_w<BX_TYPE_Q6_K>(const RawW<BX_TYPE_Q6_K>& 
 }
 #pragma clang fp contract(on)
 
-// Tile t of T (tiles of M fastest within a weight column) for block b: the
-// dispatcher deals blocks to the 8 XCDs round-robin, so XCD x receives
-// blocks x, x+8, ...; those are given the x-th contiguous run of tiles.
-__device__ __forceinline__ int xcd_tile(int b, int T) {
-    const int x = b & 7, i = b >> 3, per = T >> 3, rem = T & 7;
-    return (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + i;
-}
-
-// What a tile launch computes.  Up to three weights share the activation
-// rows X (q / k / v): member i has N[i] output columns in Y[i], tiles_n[i]
-// column tiles; a block's tile index runs over the members' column tiles in
-// order.  EPI_STORE writes Y = f16(acc + bias); EPI_RESID adds f16(acc) to
-// the FP32 residual H[M, N[0]]; EPI_SWIGLU computes gate (W[0]) and up (W[1])
-// columns of the same tile and writes Y[0] = f16(f16(silu(f16(gate))) *
-// f16(up)), the values the separate linear, silu and mul kernels give.
-enum : int { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2 };
-struct TileJob {
-    const void* W[3];
-    uint16_t* Y[3];
-    int N[3];
-    int tiles_n[3];
-    int members;
-    int tiles_m;
-    float* H;
-};
-
 // NW wavefronts (4 or 8) as (NW/2) x 2 over the block tile.
 template <int FMT, int TBM, int TBN, int NW, int EPI>
 __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(TileJob job, const uint16_t* __restrict__ X,
@@ -528,17 +504,19 @@ int gemm_tiles_typed(int wtype, const TileJob& job, const uint16_t* bias, const 
 }  // namespace
 
 bool gemm_tiles_ok(int M, int K);
+bool gemm_quant_ok(int wtype, const TileJob& job, const uint16_t* X, int M, int K);
+int gemm_quant(int wtype, int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, void* ws,
+               size_t wsb, hipStream_t st);
 
 int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, uint16_t* Y, int M, int N, int K,
-             hipStream_t st) {
-    if (gemm_tiles_ok(M, K)) {
-        TileJob job{};
-        job.W[0] = W;
-        job.Y[0] = Y;
-        job.N[0] = N;
-        job.members = 1;
-        return gemm_tiles_typed<EPI_STORE>(wtype, job, bias, X, M, K, st);
-    }
+             void* ws, size_t wsb, hipStream_t st) {
+    TileJob job{};
+    job.W[0] = W;
+    job.Y[0] = Y;
+    job.N[0] = N;
+    job.members = 1;
+    if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_STORE, job, bias, X, M, K, ws, wsb, st);
+    if (gemm_tiles_ok(M, K)) return gemm_tiles_typed<EPI_STORE>(wtype, job, bias, X, M, K, st);
     const dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
     if (grid.y > 65535) return fail(BX_EINVAL, "gemm: M too large");
     switch (wtype) {
@@ -554,7 +532,7 @@ int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, 
 bool gemm_tiles_ok(int M, int K) { return M >= 128 && K % TK == 0; }
 
 int gemm_group_f16(int wtype, int members, const void* const* W, uint16_t* const* Y, const int* N,
-                   const uint16_t* X, int M, int K, hipStream_t st) {
+                   const uint16_t* X, int M, int K, void* ws, size_t wsb, hipStream_t st) {
     TileJob job{};
     job.members = members;
     for (int i = 0; i < members; ++i) {
@@ -562,26 +540,30 @@ int gemm_group_f16(int wtype, int members, const void* const* W, uint16_t* const
         job.Y[i] = Y[i];
         job.N[i] = N[i];
     }
+    if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_STORE, job, nullptr, X, M, K, ws, wsb, st);
     return gemm_tiles_typed<EPI_STORE>(wtype, job, nullptr, X, M, K, st);
 }
 
-int gemm_resid_f16(int wtype, const void* W, const uint16_t* X, float* H, int M, int N, int K, hipStream_t st) {
+int gemm_resid_f16(int wtype, const void* W, const uint16_t* X, float* H, int M, int N, int K, void* ws, size_t wsb,
+                   hipStream_t st) {
     TileJob job{};
     job.W[0] = W;
     job.N[0] = N;
     job.members = 1;
     job.H = H;
+    if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_RESID, job, nullptr, X, M, K, ws, wsb, st);
     return gemm_tiles_typed<EPI_RESID>(wtype, job, nullptr, X, M, K, st);
 }
 
 int gemm_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X, uint16_t* Y, int M, int F, int K,
-                    hipStream_t st) {
+                    void* ws, size_t wsb, hipStream_t st) {
     TileJob job{};
     job.W[0] = Wg;
     job.W[1] = Wu;
     job.Y[0] = Y;
     job.N[0] = F;
     job.members = 1;
+    if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_SWIGLU, job, nullptr, X, M, K, ws, wsb, st);
     return gemm_tiles_typed<EPI_SWIGLU>(wtype, job, nullptr, X, M, K, st);
 }
 

@@ -14,12 +14,13 @@ namespace bx {
 
 bool gemm_tiles_ok(int M, int K);
 int gemm_group_f16(int wtype, int members, const void* const* W, uint16_t* const* Y, const int* N,
-                   const uint16_t* X, int M, int K, hipStream_t st);
-int gemm_resid_f16(int wtype, const void* W, const uint16_t* X, float* H, int M, int N, int K, hipStream_t st);
+                   const uint16_t* X, int M, int K, void* ws, size_t wsb, hipStream_t st);
+int gemm_resid_f16(int wtype, const void* W, const uint16_t* X, float* H, int M, int N, int K, void* ws, size_t wsb,
+                   hipStream_t st);
 int gemm_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X, uint16_t* Y, int M, int F, int K,
-                    hipStream_t st);
+                    void* ws, size_t wsb, hipStream_t st);
 int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, uint16_t* Y, int M, int N, int K,
-             hipStream_t st);
+             void* ws, size_t wsb, hipStream_t st);
 int gemv_mfma(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, uint16_t* Y, int M, int N, int K,
               void* ws, size_t wsb, hipStream_t st);
 // One-row GEMV with K split over a workgroup's wavefronts (K 24576 or 32768):
@@ -550,7 +551,7 @@ extern "C" int bx_linear_f16(int wtype, const void* W, const uint16_t* bias, con
         const int rc = bx::gemv_mfma_split(wtype, W, bias, X, Y, M, N, K, ws, ws_bytes, st);
         if (rc != BX_EUNSUPPORTED) return rc;
     }
-    return bx::gemm_f16(wtype, W, bias, X, Y, M, N, K, st);
+    return bx::gemm_f16(wtype, W, bias, X, Y, M, N, K, ws, ws_bytes, st);
 }
 
 extern "C" int bx_linear_tiles_ok(int M, int K) { return (bx::gemm_tiles_ok(M, K) || bx::fused_gemv_ok(M, K)) ? 1 : 0; }
@@ -566,7 +567,7 @@ extern "C" int bx_linear_group_f16(int wtype, int n, const void* const* W, uint1
         return bx::gemv_mfma_group(wtype, n, W, Y, N, X, M, K, ws, ws_bytes, bx::as_stream(stream));
     if (!bx::gemm_tiles_ok(M, K))
         return bx::fail(BX_EUNSUPPORTED, "linear_group: needs 3 <= M <= 16 with K % 256 == 0, or M >= 128 with K % 64 == 0");
-    return bx::gemm_group_f16(wtype, n, W, Y, N, X, M, K, bx::as_stream(stream));
+    return bx::gemm_group_f16(wtype, n, W, Y, N, X, M, K, ws, ws_bytes, bx::as_stream(stream));
 }
 
 extern "C" int bx_linear_residual_f16(int wtype, const void* W, const uint16_t* X, float* H, int M, int N, int K,
@@ -576,7 +577,7 @@ extern "C" int bx_linear_residual_f16(int wtype, const void* W, const uint16_t* 
     if (bx::fused_gemv_ok(M, K)) return bx::gemv_mfma_resid(wtype, W, X, H, M, N, K, ws, ws_bytes, bx::as_stream(stream));
     if (!bx::gemm_tiles_ok(M, K))
         return bx::fail(BX_EUNSUPPORTED, "linear_residual: needs 3 <= M <= 16 with K % 256 == 0, or M >= 128 with K % 64 == 0");
-    return bx::gemm_resid_f16(wtype, W, X, H, M, N, K, bx::as_stream(stream));
+    return bx::gemm_resid_f16(wtype, W, X, H, M, N, K, ws, ws_bytes, bx::as_stream(stream));
 }
 
 extern "C" int bx_linear_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X, uint16_t* Y, int M,
@@ -587,7 +588,7 @@ extern "C" int bx_linear_swiglu_f16(int wtype, const void* Wg, const void* Wu, c
         return bx::gemv_mfma_swiglu(wtype, Wg, Wu, X, Y, M, F, K, ws, ws_bytes, bx::as_stream(stream));
     if (!bx::gemm_tiles_ok(M, K))
         return bx::fail(BX_EUNSUPPORTED, "linear_swiglu: needs 3 <= M <= 16 with K % 256 == 0, or M >= 128 with K % 64 == 0");
-    return bx::gemm_swiglu_f16(wtype, Wg, Wu, X, Y, M, F, K, bx::as_stream(stream));
+    return bx::gemm_swiglu_f16(wtype, Wg, Wu, X, Y, M, F, K, ws, ws_bytes, bx::as_stream(stream));
 }
 
 // Decode-batch forms with the residual RMSNorm carried between launches (3 <=

@@ -34,6 +34,7 @@
 #include <mutex>
 #include <utility>
 
+#include "gemm_job.h"
 #include "gemv_core.h"
 
 namespace bx {
@@ -498,19 +499,12 @@ constexpr int kSplThr = 256;
 constexpr int kSplWav = kSplThr / 64;
 constexpr int kSplMaxCps = 3;                    // chunks per slice
 constexpr int kSplMaxSlices = 64;                // K up to 49152
-constexpr int64_t kSplFloats = 16ll << 20;       // partials: 64 MB
-constexpr int kSplGroups = 4096;                 // tile groups of one launch
-
-constexpr size_t kSplCntBytes = (size_t)kSplGroups * 8;
 
 }  // namespace
 }  // namespace bx
 
 namespace bx {
 namespace {
-
-// Cache policy of the partials' buffer stores and loads: sc1, device scope.
-constexpr int kSc1 = 16;
 
 // Workgroup barrier for LDS data only: loads of global memory still in flight
 // stay in flight (__syncthreads() would wait for every one of them).

@@ -80,8 +80,9 @@ int bx_dequant_to_f32(int type, const void* carrier, float* dst, int64_t rows, i
 
 /* Workspace of the linear entry points below (no counterpart in the
  * reference: brotensor's ops keep their scratch to themselves).  Decode
- * batches of 3..16 rows over layer-sized matrices split K across
- * workgroups; their partial sums and per-tile-group counters live in `ws`
+ * batches of 3..16 rows over layer-sized matrices, and 17 rows and more where
+ * the output tiles would leave CUs idle, split K across workgroups; their
+ * partial sums and per-tile(-group) counters live in `ws`
  * (bx_linear_workspace_bytes() bytes: 32 KB of counters, 64 MB of FP32
  * partials), which the caller allocates and clears once with
  * bx_linear_workspace_init before its first use.  Every launch leaves the
