@@ -16,8 +16,10 @@
 //    contiguous run of tiles that share weight columns in its own L2.
 //  - gemm_kernel<FMT> (other shapes): 64x64 block tile, K step 32, 4
 //    wavefronts each a 32x32 quadrant of 16x16x16 MFMAs.
-// Quantized weights with K a multiple of 256 and 16-byte aligned operands run
-// gemm_quant.hip instead, at any M above 16 (gemm_quant_ok).
+// They serve what the LDS-DMA kernels leave: quantized weights with K a
+// multiple of 256 run gemm_quant.hip, FP16 weights with K a multiple of 64
+// gemm_f16.hip, at any M above 16 with 16-byte aligned operands
+// (gemm_quant_ok, gemm_f16_ok).
 #include "carrier_layout.h"
 #include "gemm_job.h"
 
@@ -507,6 +509,8 @@ bool gemm_tiles_ok(int M, int K);
 bool gemm_quant_ok(int wtype, const TileJob& job, const uint16_t* X, int M, int K);
 int gemm_quant(int wtype, int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, void* ws,
                size_t wsb, hipStream_t st);
+bool gemm_f16_ok(const TileJob& job, const uint16_t* X, int M, int K);
+int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st);
 
 int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, uint16_t* Y, int M, int N, int K,
              void* ws, size_t wsb, hipStream_t st) {
@@ -516,6 +520,7 @@ int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, 
     job.N[0] = N;
     job.members = 1;
     if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_STORE, job, bias, X, M, K, ws, wsb, st);
+    if (wtype == BX_TYPE_F16 && gemm_f16_ok(job, X, M, K)) return gemm_f16_tiles(EPI_STORE, job, bias, X, M, K, st);
     if (gemm_tiles_ok(M, K)) return gemm_tiles_typed<EPI_STORE>(wtype, job, bias, X, M, K, st);
     const dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
     if (grid.y > 65535) return fail(BX_EINVAL, "gemm: M too large");
@@ -541,6 +546,7 @@ int gemm_group_f16(int wtype, int members, const void* const* W, uint16_t* const
         job.N[i] = N[i];
     }
     if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_STORE, job, nullptr, X, M, K, ws, wsb, st);
+    if (wtype == BX_TYPE_F16 && gemm_f16_ok(job, X, M, K)) return gemm_f16_tiles(EPI_STORE, job, nullptr, X, M, K, st);
     return gemm_tiles_typed<EPI_STORE>(wtype, job, nullptr, X, M, K, st);
 }
 
@@ -552,6 +558,7 @@ int gemm_resid_f16(int wtype, const void* W, const uint16_t* X, float* H, int M,
     job.members = 1;
     job.H = H;
     if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_RESID, job, nullptr, X, M, K, ws, wsb, st);
+    if (wtype == BX_TYPE_F16 && gemm_f16_ok(job, X, M, K)) return gemm_f16_tiles(EPI_RESID, job, nullptr, X, M, K, st);
     return gemm_tiles_typed<EPI_RESID>(wtype, job, nullptr, X, M, K, st);
 }
 
@@ -564,6 +571,7 @@ int gemm_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X
     job.N[0] = F;
     job.members = 1;
     if (gemm_quant_ok(wtype, job, X, M, K)) return gemm_quant(wtype, EPI_SWIGLU, job, nullptr, X, M, K, ws, wsb, st);
+    if (wtype == BX_TYPE_F16 && gemm_f16_ok(job, X, M, K)) return gemm_f16_tiles(EPI_SWIGLU, job, nullptr, X, M, K, st);
     return gemm_tiles_typed<EPI_SWIGLU>(wtype, job, nullptr, X, M, K, st);
 }
 
