@@ -105,6 +105,7 @@ HIP_SYMBOLS = {
                                   vp]),
     "bx_persist_ws_init": (C.c_int, [C.POINTER(DecodeDimsC), vp, vp]),
     "bx_persist_status": (C.c_int, [vp, C.POINTER(C.c_uint32)]),
+    "bx_persist_status_async": (C.c_int, [vp, vp, vp]),
     "bx_persist_trace": (C.c_int, [vp, C.c_int]),
     "bx_argmax_workspace_bytes": (C.c_size_t, [i64]),
     "bx_argmax_f16": (C.c_int, [vp, i64, vp, vp, vp]),

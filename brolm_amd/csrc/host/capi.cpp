@@ -28,6 +28,7 @@ struct brolm_qwen3 {
     std::unique_ptr<brolm::mistral3::TextModel> mistral;
     std::unique_ptr<brolm::llm2vec::Encoder> encoder;
     brolm::detail::DenseDecoder* core = nullptr;
+    brotensor::Tensor last;   // one row of logits, kept: a step allocates nothing
 };
 
 struct brolm_tokenizer {
@@ -81,10 +82,7 @@ void from_cfg(const brolm::qwen::Qwen3Config& q, brolm_qwen3_config* c) {
     c->max_position_embeddings = q.max_position_embeddings;
 }
 
-void to_host_f32(const brotensor::Tensor& t, float* dst) {
-    const std::vector<float> v = t.to_host_vector();
-    std::memcpy(dst, v.data(), v.size() * sizeof(float));
-}
+void to_host_f32(const brotensor::Tensor& t, float* dst) { t.copy_to_host_f32(dst); }
 
 brolm::qwen::Qwen3Model& model_of(brolm_qwen3* m) {
     if (!m || !m->core) throw std::runtime_error("null model handle");
@@ -476,9 +474,8 @@ int brolm_qwen3_truncate_slot(brolm_qwen3* m, int slot, int len) {
 }
 int brolm_qwen3_prefill_slot(brolm_qwen3* m, int slot, const int32_t* ids, int L, float* logits) {
     return guard([&] {
-        brotensor::Tensor lg;
-        core_of(m).prefill_slot(slot, ids, L, lg);
-        if (logits) to_host_f32(lg, logits);
+        core_of(m).prefill_slot(slot, ids, L, m->last);
+        if (logits) to_host_f32(m->last, logits);
     });
 }
 int brolm_qwen3_forward_batch(brolm_qwen3* m, const int32_t* ids, const int32_t* slots, int M, float* logits) {
@@ -514,9 +511,8 @@ int brolm_qwen3_forward(brolm_qwen3* m, const int32_t* ids, int L, float* logits
 
 int brolm_qwen3_forward_last(brolm_qwen3* m, const int32_t* ids, int L, float* logits) {
     return guard([&] {
-        brotensor::Tensor lg;
-        core_of(m).forward_last(ids, L, lg);
-        if (logits) to_host_f32(lg, logits);
+        core_of(m).forward_last(ids, L, m->last);
+        if (logits) to_host_f32(m->last, logits);
     });
 }
 

@@ -63,7 +63,7 @@ struct DecodeGraphSession {
     int32_t* scal = nullptr;
     uint16_t* logits = nullptr;
     void* argmax_ws = nullptr;
-    int32_t* pinned = nullptr;  // host staging {tok, pos, next, count}
+    int32_t* pinned = nullptr;  // host staging {tok, pos, next, count}, then the abort words {flag, site}
     hipEvent_t staged = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -728,7 +728,7 @@ DecodeGraphSession& DenseDecoder::session_() {
     hipx::check(hipMalloc(reinterpret_cast<void**>(&s->logits), static_cast<std::size_t>(cfg_.vocab_size) * 2),
                 "hipMalloc logits");
     hipx::check(hipMalloc(&s->argmax_ws, bx_argmax_workspace_bytes(cfg_.vocab_size)), "hipMalloc argmax ws");
-    hipx::check(hipHostMalloc(reinterpret_cast<void**>(&s->pinned), 4 * sizeof(int32_t), hipHostMallocDefault),
+    hipx::check(hipHostMalloc(reinterpret_cast<void**>(&s->pinned), 6 * sizeof(int32_t), hipHostMallocDefault),
                 "hipHostMalloc");
     hipx::check(hipEventCreateWithFlags(&s->staged, hipEventDisableTiming), "hipEventCreate");
     // no captured graph under a profiler tool: a graph launch under
@@ -792,11 +792,11 @@ static void stage_step(DecodeGraphSession& s, int32_t token, int32_t pos) {
 // s.aborted tells the caller to redo the steps it enqueued since its last
 // check (they rewrite the same cache rows).
 static bool persist_gave_up(DecodeGraphSession& s) {
+    auto* words = reinterpret_cast<uint32_t*>(s.pinned + 4);
+    hipx::bx(bx_persist_status_async(s.pws, words, hipx::stream()), "persist status");
     hipx::check(hipStreamSynchronize(hipx::stream()), "hipStreamSynchronize");
-    uint32_t site = 0;
-    const int st = bx_persist_status(s.pws, &site);
-    if (st < 0) hipx::bx(st, "persist status");
-    if (st == 0) return false;
+    if (words[0] == 0) return false;
+    const uint32_t site = words[1];
     hipx::bx(bx_persist_ws_init(&s.dims, s.pws, hipx::stream()), "persist ws init");
     hipx::check(hipStreamSynchronize(hipx::stream()), "hipStreamSynchronize");
     std::fprintf(stderr, "brolm: persistent decode step gave up waiting at site %u; the per-stage graph runs from here on\n",

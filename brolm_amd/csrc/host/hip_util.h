@@ -28,5 +28,7 @@ std::size_t linear_ws_bytes();
 // Stream-ordered copies; the host side waits (synchronous semantics).
 void h2d(void* dst, const void* src, std::size_t n);
 void d2h(void* dst, const void* src, std::size_t n);
+// n FP16 device values as FP32 in host memory, after the stream's work so far.
+void d2h_f16_as_f32(float* dst, const void* src, std::size_t n);
 
 }  // namespace hipx

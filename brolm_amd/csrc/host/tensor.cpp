@@ -333,12 +333,21 @@ std::vector<std::uint16_t> Tensor::to_host_vector_fp16() const {
 }
 
 std::vector<float> Tensor::to_host_vector() const {
+    std::vector<float> out(static_cast<std::size_t>(size()));
+    copy_to_host_f32(out.data());
+    return out;
+}
+
+void Tensor::copy_to_host_f32(float* out) const {
     const std::size_t n = static_cast<std::size_t>(size());
-    std::vector<float> out(n);
     if (dtype == Dtype::FP32) {
-        if (device == Device::CPU) std::memcpy(out.data(), data, n * 4);
-        else hipx::d2h(out.data(), data, n * 4);
-        return out;
+        if (device == Device::CPU) std::memcpy(out, data, n * 4);
+        else hipx::d2h(out, data, n * 4);
+        return;
+    }
+    if (dtype == Dtype::FP16 && device != Device::CPU) {
+        hipx::d2h_f16_as_f32(out, data, n);
+        return;
     }
     if (dtype == Dtype::FP16 || dtype == Dtype::BF16) {
         std::vector<std::uint16_t> bits(n);
@@ -346,7 +355,7 @@ std::vector<float> Tensor::to_host_vector() const {
         else hipx::d2h(bits.data(), data, n * 2);
         for (std::size_t i = 0; i < n; ++i)
             out[i] = dtype == Dtype::FP16 ? fp16_bits_to_fp32(bits[i]) : bf16_bits_to_fp32(bits[i]);
-        return out;
+        return;
     }
     throw std::runtime_error(std::string("to_host_vector: unsupported dtype ") + dtype_name(dtype));
 }

@@ -2037,6 +2037,12 @@ extern "C" int bx_persist_status(const void* ws, uint32_t* site) {
     return c[0] ? 1 : 0;
 }
 
+extern "C" int bx_persist_status_async(const void* ws, uint32_t* out2, void* stream) {
+    if (!ws || !out2) return bx::fail(BX_EINVAL, "persist_status_async: null argument");
+    return bx::hip_check(hipMemcpyAsync(out2, ws, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, bx::as_stream(stream)),
+                         "persist_status_async: copy");
+}
+
 extern "C" int bx_persist_trace(uint64_t* buf_dev, int slots_per_wg) {
     if (buf_dev && slots_per_wg < bx::p2::kTraceSlots)
         return bx::fail(BX_EINVAL, "persist_trace: need 1024 slots per workgroup");

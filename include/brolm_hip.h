@@ -357,6 +357,10 @@ int bx_persist_step(const bx_decode_dims* d, int n_layers, const bx_decode_layer
                     const uint16_t* embed, const uint16_t* final_norm, const void* lm_head, const float* cos_tab,
                     const float* sin_tab, int32_t* scal, uint16_t* logits, void* ws, uint32_t epoch, void* stream);
 int bx_persist_status(const void* ws, uint32_t* site);
+/* The same words {flag, site} copied to out2 (host, pinned for an asynchronous
+ * copy) in stream order: valid once the stream has been waited for, with no
+ * copy of their own to wait for. */
+int bx_persist_status_async(const void* ws, uint32_t* out2, void* stream);
 /* Debug timing (no counterpart in the reference): while buf_dev is non-null,
  * every later bx_persist_step writes the device wall clock (wall_clock64, the
  * constant-rate counter) at each stage boundary of each workgroup into

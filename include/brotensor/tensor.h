@@ -76,6 +76,7 @@ public:
 
     void copy_to_host_fp16(std::uint16_t* dst) const;   // FP16 tensors
     std::vector<float> to_host_vector() const;           // FP32 / FP16 / BF16 -> FP32
+    void copy_to_host_f32(float* dst) const;             // the same into a caller's buffer of size() values
     std::vector<std::uint16_t> to_host_vector_fp16() const;
     void* host_raw_mut();
     const void* host_raw() const;
