@@ -354,6 +354,17 @@ int attn_keys_per_split(int L, int n_kv, int valid_len) {
     return kps;
 }
 
+// The workspace is sized for n_kv = 1 (most splits).
+int attn_ws_splits(int L, int valid_len) {
+    const int kps = attn_keys_per_split(L, 1, valid_len);
+    return (valid_len + kps - 1) / kps;
+}
+
+int attn_combine(const float* ws, int n_q, int L, int hd, int S, uint16_t* out, hipStream_t st) {
+    attn_combine_kernel<<<dim3(n_q, L), 128, combine_lds(S), st>>>(ws, n_q, hd, S, out);
+    return launch_check("attention combine");
+}
+
 }  // namespace bx
 
 using namespace bx;
@@ -362,10 +373,7 @@ extern "C" {
 
 size_t bx_attention_workspace_bytes(int L, int n_q, int hd, int valid_len) {
     if (L <= 0 || n_q <= 0 || hd <= 0 || valid_len <= 0) return 0;
-    // Worst case over n_kv >= 1 is n_kv = 1 (most splits).
-    const int kps = attn_keys_per_split(L, 1, valid_len);
-    const int S = (valid_len + kps - 1) / kps;
-    return (size_t)L * n_q * S * (hd + 2) * sizeof(float);
+    return (size_t)L * n_q * attn_ws_splits(L, valid_len) * (hd + 2) * sizeof(float);
 }
 
 int bx_attention_decode_f16(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q,
@@ -377,7 +385,7 @@ int bx_attention_decode_f16(const uint16_t* q, const uint16_t* Kc, const uint16_
     if (hd <= 0 || hd % 8 || hd > 256) return fail(BX_EUNSUPPORTED, "attention: head_dim must be a multiple of 8, <= 256");
     if (valid_len < L) return fail(BX_EINVAL, "attention: valid_len < L");
     if (attn_mfma_supported(L, hd, softcap, window, nullptr))
-        return attn_mfma(q, Kc, Vc, L, valid_len, n_q, n_kv, hd, 0, out, as_stream(stream));
+        return attn_mfma(q, Kc, Vc, L, valid_len, n_q, n_kv, hd, 0, workspace, out, as_stream(stream));
     if (!attn_span_ok(valid_len, n_kv, hd)) return fail(BX_EUNSUPPORTED, "attention: cache rows span 2 GiB or more");
     AttnArgs a{};
     a.q = q; a.Kc = Kc; a.Vc = Vc; a.mask = nullptr;
@@ -403,7 +411,7 @@ int bx_attention_gqa_f16(const uint16_t* q, const uint16_t* K, const uint16_t* V
         return fail(BX_EUNSUPPORTED, "attention_gqa: head_dim must be a multiple of 8, <= 256");
     if (causal && n_keys < L) return fail(BX_EINVAL, "attention_gqa: causal with fewer keys than rows");
     if (attn_mfma_supported(L, hd, 0.f, 0, nullptr))
-        return attn_mfma(q, K, V, L, n_keys, n_q, n_kv, hd, causal ? 0 : 1, out, as_stream(stream));
+        return attn_mfma(q, K, V, L, n_keys, n_q, n_kv, hd, causal ? 0 : 1, workspace, out, as_stream(stream));
     if (!attn_span_ok(n_keys, n_kv, hd)) return fail(BX_EUNSUPPORTED, "attention_gqa: keys span 2 GiB or more");
     AttnArgs a{};
     a.q = q; a.Kc = K; a.Vc = V; a.mask = nullptr;

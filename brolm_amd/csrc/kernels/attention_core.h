@@ -27,8 +27,14 @@ struct AttnArgs {
 
 // Flash attention on MFMA for L >= 16 query rows (attention_mfma.hip): head
 // dims 64 and 128, no softcap / window / key mask.
+// ws: the caller's bx_attention_workspace_bytes(L, n_q, hd, valid_len).
 bool attn_mfma_supported(int L, int hd, float softcap, int window, const float* mask);
 int attn_mfma(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
-              int hd, int bidir, uint16_t* out, hipStream_t st);
+              int hd, int bidir, void* ws, uint16_t* out, hipStream_t st);
+
+// Records per (row, query head) that bx_attention_workspace_bytes has room for.
+int attn_ws_splits(int L, int valid_len);
+// Merge S records per (row, query head) of ws [L][n_q][S][hd + 2] into out.
+int attn_combine(const float* ws, int n_q, int L, int hd, int S, uint16_t* out, hipStream_t st);
 
 }  // namespace bx

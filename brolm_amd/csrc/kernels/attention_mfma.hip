@@ -4,296 +4,378 @@
 // at positions valid_len - L ...) and flash_attention_gqa_forward
 // (dense_decoder.cpp:737-745, causal or bidirectional).
 //
-// Block = 4 wavefronts over one KV head: each wavefront holds NF = GB x R
-// query fragments of 16 rows (GB query heads of the group, R row groups), so
-// every K / V^T fragment it reads from LDS feeds NF MFMAs.  Keys stream in
-// tiles of 64 through LDS (K as stored, V transposed so both MFMA operands
-// are contiguous reads), double buffered: the next tile's global loads are
-// issued before this tile's MFMAs.  Per key tile, on v_mfma_f32_16x16x32_f16:
-//   S^T = K Q^T     (16 keys x 16 queries per fragment; the query fragments
-//                    stay in registers for the whole key loop)
-//   online softmax  (base-2 exponent, running max / sum per query in FP32;
-//                    the four lanes holding a query combine by ds_bpermute;
-//                    the running max moves lazily, only by more than 2^8,
-//                    and tiles below the diagonal skip the causal mask)
-//   O^T += V^T P^T  (P converted to FP16 in registers: the S^T layout is
-//                    the B operand's, with the 8 keys of a k-slot group in a
-//                    fixed permutation that the V^T reads follow; O^T keeps
-//                    each query in one lane, so the rescale needs no shuffle)
-// Row tiles are issued latest-first (they see the most keys).  Results
-// differ from the split-K kernel by FP16 rounding of P (relative 2^-11).
+// A workgroup of four wavefronts works on one KV head.  A wavefront holds 32
+// query rows of one head in registers; 4 / KS wavefronts take different rows
+// and heads of the group (they share every key tile), KS wavefronts the same
+// rows over different keys of a tile, merged at the end (small problems, where
+// the serial walk over the keys is what takes the time).  Keys and values come
+// in tiles by LDS-DMA, double buffered, rows as stored, 16-byte chunks
+// XOR-swizzled by the key.  Per 32 keys, on v_mfma_f32_32x32x16_f16:
+//   S^T = K Q^T     (a lane holds 16 of the 32 keys of its query)
+//   online softmax  (base-2 exponent, running max per query in FP32, moved only
+//                    when some tile max exceeds it by more than 2^8; a lane
+//                    sums its own keys, the halves of a query add at the end)
+//   O^T += V^T P^T  (P to FP16 in registers: the S^T layout is the B operand's
+//                    with the keys of a k-slot group in a fixed order; V^T
+//                    comes out of the row-major tile by transposing LDS reads,
+//                    four keys of a column each, in that order)
+//
+// What bounds it: per 32 keys of a wavefront about 512 cycles of MFMA and 450
+// of softmax arithmetic (half of them the exponentials, at quarter rate),
+// overlapped by the two wavefronts of each SIMD (two workgroups per CU), and
+// the LDS reads of both operands (16 KB, which is why one fragment of K feeds
+// 32 queries and not 16).  Measured against 16-row fragments with tiles staged
+// through registers and V transposed on its way into LDS: 2048 causal rows of
+// 32 / 8 heads of 128 100.5 -> 54.0 us (640 TFLOP/s), 500 rows bidirectional
+// of 16 heads 19.8 -> 10.4 us, 1024 rows after 1500 of 32 heads 102 -> 52 us,
+// 64 rows after 2000 of 16 heads 62 -> 13 us.
+#include <algorithm>
+
 #include "attention_core.h"
+#include "gemm_job.h"
 
 namespace bx {
 namespace {
 
 typedef _Float16 fa_h8 __attribute__((ext_vector_type(8)));
-typedef float fa_f4 __attribute__((ext_vector_type(4)));
+typedef _Float16 fa_h4 __attribute__((ext_vector_type(4)));
+typedef short fa_s4 __attribute__((ext_vector_type(4)));
+typedef float fa_f16 __attribute__((ext_vector_type(16)));
 
-constexpr int kFaKeys = 64;
+constexpr int kFaThreads = 256;
 
-template <int HD>
+template <int HD, int KS>
 struct FaShape {
-    static constexpr int KROW = HD + 8;                  // K tile row stride (halves): rows 4 banks apart
-    static constexpr int VROW = kFaKeys + 8;             // V^T row stride (halves)
-    static constexpr int CH = HD / 8;                    // 16-byte chunks per key row
-    static constexpr int KRPP = 256 / CH;                // key rows one loader pass covers
-    static constexpr int KPASS = kFaKeys / KRPP;         // loader passes for K
-    static constexpr int VKP = kFaKeys / (256 / CH);     // keys per thread in the V transpose (4 or 2)
-    static constexpr int VNG = kFaKeys / VKP;            // key groups of the V transpose (16 or 32)
+    static constexpr int TK = KS == 4 ? 128 : 64;       // keys per tile
+    static constexpr int WK = TK / KS;                  // keys per wavefront and tile
+    static constexpr int NK = WK / 32;                  // 32-key fragments per wavefront and tile
+    static constexpr int RB = HD * 2;                   // bytes per key row
+    static constexpr int CH = HD / 8;                   // 16-byte chunks per key row
+    static constexpr int RPC = 1024 / RB;               // rows per copy instruction
+    static constexpr int P = TK / RPC / 4;              // copies per wavefront and tile, of K and of V
+    static constexpr int kTile = TK * RB;               // bytes of a K (or V) tile
+    static constexpr int kBuf = 2 * kTile;
+    static constexpr int kMerge = KS > 1 ? 4 * 64 * (HD / 32 * 16 + 2) * 4 : 0;   // end merge, FP32
+    static constexpr int kLds = 2 * kBuf > kMerge ? 2 * kBuf : kMerge;
+    // chunk c of key k sits at c ^ swz(k): the 16 keys a K read covers land on
+    // distinct chunks of the banks, and so do the 4 keys of a transposing read
+    static __device__ __forceinline__ int swz(int k) {
+        return CH == 16 ? ((k & 3) << 2) | ((k >> 2) & 3) : (k >> 1) & 7;
+    }
 };
 
-// Pairwise max / sum with the lanes 16 and 32 positions away (the other rows
-// holding the same query).  v_permlane16/32_swap would keep this off the LDS
-// path, but this compiler folds a swap whose two operands hold one value
-// into a copy and drops the exchange, so ds_bpermute it is.
-__device__ __forceinline__ float fa_max_rows(float v) {
-    v = fmaxf(v, __shfl_xor(v, 16));
-    return fmaxf(v, __shfl_xor(v, 32));
-}
-__device__ __forceinline__ float fa_sum_rows(float v) {
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
+// Eight halves at any 2-byte address.
+__device__ __forceinline__ fa_h8 fa_load8(const uint16_t* p) {
+    uint16_t v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = p[e];
+    return __builtin_bit_cast(fa_h8, v);
 }
 
-// GB query heads of one KV group x R fragments of 16 rows per wavefront
-// (NF = GB * R query fragments share every K / V^T fragment read from LDS);
-// 4 wavefronts stack 4 * 16 * R rows.
-template <int HD, int GB, int R>
-__global__ __launch_bounds__(256, (HD == 128 && GB * R > 2) ? 1 : 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
-                                                 const uint16_t* __restrict__ Vc, int L, int valid_len, int n_q,
-                                                 int n_kv, int bidir, uint16_t* __restrict__ out) {
-    using S = FaShape<HD>;
-    constexpr int NF = GB * R, BR = 64 * R;
-    __shared__ __align__(16) uint16_t Ks[2][kFaKeys * S::KROW];
-    __shared__ __align__(16) uint16_t Vt[2][HD * S::VROW];
+// The larger of a query's two lanes (l and l ^ 32), in both.
+__device__ __forceinline__ float fa_pair_max(float v) { return fmaxf(v, __shfl_xor(v, 32)); }
 
-    const int G = n_q / n_kv, splits = G / GB;
-    const int ntile = (L + BR - 1) / BR;
-    const int rt = ntile - 1 - (int)blockIdx.x;  // latest rows first: they see the most keys
-    const int g = (int)blockIdx.y / splits, h0 = g * G + ((int)blockIdx.y % splits) * GB;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lq = lane & 15, lg = lane >> 4;
+// AL: the operands are 16-byte aligned (out: 8); otherwise tiles go through
+// registers in 2-byte loads, and so do q and out.
+template <int HD, int KS, bool AL>
+__global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
+                                                          const uint16_t* __restrict__ Vc, int L, int valid_len,
+                                                          int n_q, int n_kv, int bidir, int gb, int mirror, int nsp,
+                                                          float* __restrict__ recs, uint16_t* __restrict__ out) {
+    using S = FaShape<HD, KS>;
+    constexpr int NK = S::NK, ND = HD / 32;
+    extern __shared__ __align__(1024) unsigned char smem[];
+
+    // block -> (row tile, head set): latest rows first (they see the most
+    // keys); blocks from `mirror` on, the second of each CU where the grid
+    // just fits two per CU, take the remaining row tiles from the lightest up
+    const int G = n_q / n_kv, splits = G / gb, ny = n_kv * splits;
+    // (sp > 1: sp blocks in turn share a row tile's key tiles)
+    const int sp = KS == 4 ? nsp : 1;
+    int b = (int)blockIdx.x / sp;
+    const int part = (int)blockIdx.x % sp;
+    if (b >= mirror) b = mirror + (int)gridDim.x - 1 - b;
+    const int rg = 4 / KS / gb, BR = 32 * rg;     // row groups and rows per workgroup
+    const int rt = (L + BR - 1) / BR - 1 - b / ny, y = b % ny;
+    const int g = y / splits;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int qw = wave / KS, kw = wave % KS;     // (rows, head) of the wavefront, its keys of a tile
+    const int head = g * G + (y % splits) * gb + qw % gb;
+    const int lq = lane & 31, lh = lane >> 5;
     const int p0 = valid_len - L;  // position of query row 0
     const int64_t qstride = (int64_t)n_q * HD, kvstride = (int64_t)n_kv * HD;
+    const int row0 = rt * BR + 32 * (qw / gb), row = row0 + lq;
     const int kend = bidir ? valid_len : min(valid_len, p0 + rt * BR + BR);
-    const int nkb = (kend + kFaKeys - 1) / kFaKeys;
+    const int nkb = (kend + S::TK - 1) / S::TK;
+    const int last_key = bidir ? valid_len - 1 : min(p0 + row, valid_len - 1);
+    // keys every query of the wavefront sees (its first row's)
+    const int all_see = bidir ? valid_len - 1 : min(p0 + row0, valid_len - 1);
+    // keys some query of the wavefront sees
+    const int any_see = bidir ? valid_len - 1 : min(p0 + row0 + 31, valid_len - 1);
 
-    // fragment f: rows row0 + 16*(f / GB) + lq of head h0 + f % GB; this
-    // lane holds query lq of each fragment (the column of S^T and O^T)
-    const int row0 = rt * BR + wave * 16 * R;
-    int last[NF];
-    fa_h8 qf[NF][HD / 32];
+    // ---- copies: wavefront w takes rows RPC (w P + j) .. of a tile
+    const uint32_t lbase = lds_addr(smem);
+    const unsigned char* const kb0 = reinterpret_cast<const unsigned char*>(Kc + (int64_t)g * HD);
+    const unsigned char* const vb0 = reinterpret_cast<const unsigned char*>(Vc + (int64_t)g * HD);
+    const int drow = lane / S::CH, dch = lane % S::CH;
+    auto issue = [&](int kb, int buf) {
+        const int k0 = kb * S::TK, left = valid_len - 1 - k0;   // keys past the end repeat the last one
+        const int64_t base = (int64_t)k0 * kvstride * 2;
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lbase + buf * S::kBuf + wave * S::P * 1024);
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const int qi = row0 + 16 * (f / GB) + lq;
-        last[f] = bidir ? valid_len - 1 : min(p0 + qi, valid_len - 1);
-        const uint16_t* qrow = q + (int64_t)min(qi, L - 1) * qstride + (int64_t)(h0 + f % GB) * HD;
-#pragma unroll
-        for (int s = 0; s < HD / 32; ++s) qf[f][s] = *reinterpret_cast<const fa_h8*>(qrow + 32 * s + 8 * lg);
-    }
-
-    // loaders: K rows kr0 + KRPP*i, chunk kc (a row per CH lanes, coalesced);
-    // V keys vq*VKP .. +VKP, chunk vc, consecutive lanes on consecutive key
-    // groups so that the transposed LDS writes of a wavefront land on
-    // consecutive banks (a lane per d-chunk instead puts 16 lanes 8 rows of
-    // V^T apart, an 8-way bank conflict on every write)
-    const int kr0 = tid / S::CH, kc = (tid % S::CH) * 8;
-    const int vq = tid % S::VNG, vc = (tid / S::VNG) * 8;
-    const uint16_t* kbase = Kc + (int64_t)g * HD;
-    const uint16_t* vbase = Vc + (int64_t)g * HD;
-    u4v kreg[S::KPASS], vreg[S::VKP];
-    auto gload = [&](int kb) {
-        const int k0 = kb * kFaKeys;
-#pragma unroll
-        for (int i = 0; i < S::KPASS; ++i) {
-            const int key = min(k0 + kr0 + S::KRPP * i, valid_len - 1);
-            kreg[i] = ldg16(kbase + (int64_t)key * kvstride + kc);
-        }
-#pragma unroll
-        for (int i = 0; i < S::VKP; ++i) {
-            const int key = min(k0 + vq * S::VKP + i, valid_len - 1);
-            vreg[i] = ldg16(vbase + (int64_t)key * kvstride + vc);
-        }
-    };
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < S::KPASS; ++i)
-            *reinterpret_cast<u4v*>(&Ks[buf][(kr0 + S::KRPP * i) * S::KROW + kc]) = kreg[i];
-        // V^T[d][key]: the VKP keys of this thread for each of its 8 d values
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            uint32_t hv[S::VKP];
-#pragma unroll
-            for (int i = 0; i < S::VKP; ++i) hv[i] = (vreg[i][e >> 1] >> (16 * (e & 1))) & 0xffff;
-            uint16_t* dst = &Vt[buf][(vc + e) * S::VROW + vq * S::VKP];
-            if constexpr (S::VKP == 4) {
-                u2v w;
-                w.x = hv[0] | (hv[1] << 16);
-                w.y = hv[2] | (hv[3] << 16);
-                *reinterpret_cast<u2v*>(dst) = w;
+        for (int j = 0; j < S::P; ++j) {
+            const int r = S::RPC * (wave * S::P + j) + drow;
+            const uint32_t off = (uint32_t)min(r, left) * (uint32_t)(kvstride * 2) + (uint32_t)((dch ^ S::swz(r)) * 16);
+            if constexpr (AL) {
+                dma16(off, kb0 + base, dst + j * 1024);
+                dma16(off, vb0 + base, dst + S::kTile + j * 1024);
             } else {
-                *reinterpret_cast<uint32_t*>(dst) = hv[0] | (hv[1] << 16);
+                unsigned char* const d = smem + buf * S::kBuf + (wave * S::P + j) * 1024 + lane * 16;
+                *reinterpret_cast<fa_h8*>(d) = fa_load8(reinterpret_cast<const uint16_t*>(kb0 + base + off));
+                *reinterpret_cast<fa_h8*>(d + S::kTile) = fa_load8(reinterpret_cast<const uint16_t*>(vb0 + base + off));
             }
         }
     };
 
-    // O^T fragments: o[j][f] holds d = 16j + 4*lg + r (r = 0..3) for query lq of fragment f
-    fa_f4 o[HD / 16][NF];
+    auto tile_wait = [] {   // this tile's readers are done and the next one is there
+        if constexpr (AL)
+            wait_vm_barrier<0>();
+        else
+            __syncthreads();
+    };
+
+    // the query rows: B operand, lane l holds query l % 32, d 16 s + 8 (l / 32) ..
+    fa_h8 qf[HD / 16];
+    {
+        const uint16_t* qrow = q + (int64_t)min(row, L - 1) * qstride + (int64_t)head * HD + 8 * lh;
 #pragma unroll
-    for (int j = 0; j < HD / 16; ++j)
+        for (int s = 0; s < HD / 16; ++s)
+            qf[s] = AL ? *reinterpret_cast<const fa_h8*>(qrow + 16 * s) : fa_load8(qrow + 16 * s);
+        // waited for here: left to their first use, inside the loop, the wait
+        // would also cover the tile copies just issued there, every iteration
 #pragma unroll
-        for (int f = 0; f < NF; ++f) o[j][f] = (fa_f4){0.f, 0.f, 0.f, 0.f};
-    float m[NF], l[NF];  // running max (base-2 units) and sum per fragment query
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        m[f] = -INFINITY;
-        l[f] = 0.f;
+        for (int s = 0; s < HD / 16; ++s) asm volatile("" : "+v"(qf[s]));
     }
+    fa_f16 o[ND];   // O^T: d = 32 j + 8 (r / 4) + 4 lh + r % 4 of query lq
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[j][r] = 0.f;
+    float m = -INFINITY, l = 0.f;   // running max (base-2 units), sum over this lane's keys
     const float sl2 = 1.4426950408889634f / sqrtf((float)HD);
-    // the smallest last-visible key over the block's rows (its first row)
-    const int first_last = bidir ? valid_len - 1 : min(p0 + rt * BR, valid_len - 1);
 
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int kb = 0; kb < nkb; ++kb) {
-        const int cur = kb & 1;
-        if (kb + 1 < nkb) gload(kb + 1);
+    // LDS addresses: K rows of 32 keys (A operand: lane l holds key l % 32,
+    // d 16 s + 8 (l / 32)); transposing reads of V (lane i of a group of 16
+    // reads four columns of key i / 4 and receives column i of four keys)
+    const int krow = kw * S::WK + lq;
+    const int ka = krow * S::RB, kx = S::swz(krow) ^ lh;   // (2 s + lh) ^ swz = 2 s ^ kx
+    const int ti = lane & 15, tg = (lane >> 4) & 1;
+    const int vkey = kw * S::WK + 4 * lh + (ti >> 2), vcol = 2 * tg + ((ti & 3) >> 1), vb8 = (ti & 1) * 8;
 
-        // S^T: s[t][f] holds keys 16t + 4*lg + r for query lq of fragment f
-        fa_f4 s[4][NF];
+    const int kb_first = (int)((int64_t)nkb * part / sp), kb_end = (int)((int64_t)nkb * (part + 1) / sp);
+    if (kb_first < kb_end) issue(kb_first, 0);
+    tile_wait();
+    for (int kb = kb_first; kb < kb_end; ++kb) {
+        const int cur = (kb - kb_first) & 1;
+        if (kb + 1 < kb_end) issue(kb + 1, cur ^ 1);
+        const unsigned char* const kt = smem + cur * S::kBuf;
+        const unsigned char* const vt = kt + S::kTile;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < NK; ++t) {
+            const int key0 = kb * S::TK + kw * S::WK + 32 * t;   // 32 keys at a time
+            if (key0 > any_see) break;
+            fa_h8 kf[HD / 16];
 #pragma unroll
-            for (int f = 0; f < NF; ++f) s[t][f] = (fa_f4){0.f, 0.f, 0.f, 0.f};
+            for (int d = 0; d < HD / 16; ++d)
+                kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + t * 32 * S::RB + (((2 * d) ^ kx) << 4));
+            __builtin_amdgcn_sched_barrier(0);
+            fa_f16 s;
 #pragma unroll
-            for (int ds = 0; ds < HD / 32; ++ds) {
-                const fa_h8 a = *reinterpret_cast<const fa_h8*>(&Ks[cur][(16 * t + lq) * S::KROW + 32 * ds + 8 * lg]);
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
-                for (int f = 0; f < NF; ++f) s[t][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qf[f][ds], s[t][f], 0, 0, 0);
-            }
-        }
-        // a tile every query of the block sees in full needs no mask
-        const bool full = kb * kFaKeys + kFaKeys - 1 <= first_last;
-        const int key0 = kb * kFaKeys + 4 * lg;
+            for (int d = 0; d < HD / 16; ++d) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[d], qf[d], s, 0, 0, 0);
+            // the values are requested before the softmax that weighs them:
+            // k-slot (lh, e) of V^T holds key 16 u + 4 lh + e (e < 4) or 16 u +
+            // 8 + 4 lh + e - 4 (e >= 4)
+            fa_h8 vf[2][ND];
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            float mx = -INFINITY;
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (!full && key0 + 16 * t + r > last[f]) s[t][f][r] = -INFINITY;
-                    mx = fmaxf(mx, s[t][f][r]);
+                for (int j = 0; j < ND; ++j) {
+                    const int c = 4 * j + vcol;
+                    const int k1 = 32 * t + 16 * u + vkey, k2 = k1 + 8;
+                    const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + vb8;
+                    const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + vb8;
+                    const fa_h4 lo = __builtin_bit_cast(
+                        fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a1));
+                    const fa_h4 hi = __builtin_bit_cast(
+                        fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a2));
+                    vf[u][j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                 }
-            mx = fa_max_rows(mx) * sl2;  // the tile's max in base-2 units (sl2 > 0)
+            __builtin_amdgcn_sched_barrier(0);
+            // lane l, register r: key 8 (r / 4) + 4 lh + r % 4
+            if (key0 + 31 > all_see) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (key0 + 8 * (r >> 2) + 4 * lh + (r & 3) > last_key) s[r] = -INFINITY;
+            }
+            float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+            for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            mx = fa_pair_max(mx) * sl2;  // the tile's max in base-2 units (sl2 > 0)
             // v_exp_f32 flushes results below 2^-126 to zero: weights that
             // small (scores 87 natural units under the row max) are zero in
-            // any FP16 / FP32 sum here anyway
+            // any FP16 / FP32 sum here anyway.
             // Lazy rescale: the running max moves only when some query's tile
             // max exceeds it by more than 8 (a factor 256; P stays <= 256,
-            // well inside FP16).  Key 0 is in every query's first tile, so
-            // that tile always moves it off -inf.
-            if (__any(mx > m[f] + 8.f)) {
-                const float mnew = fmaxf(m[f], mx);
-                const float alpha = __builtin_amdgcn_exp2f(m[f] - mnew);
-                l[f] *= alpha;
+            // well inside FP16).  A query that has seen no key yet has m =
+            // -inf: its first visible tile moves it, and until then every
+            // weight is exp2(-inf - finite) = 0 (nm below).
+            if (__any(mx > m + 8.f)) {
+                const float mnew = fmaxf(m, mx);
+                const float alpha = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);
+                l *= alpha;
 #pragma unroll
-                for (int j = 0; j < HD / 16; ++j) o[j][f] *= alpha;
-                m[f] = mnew;
+                for (int j = 0; j < ND; ++j) o[j] *= alpha;
+                m = mnew;
             }
-            const float nm = -m[f];
-            float ls = 0.f;
+            const float nm = m == -INFINITY ? 0.f : -m;
+            fa_h8 pb[2];   // B operands: 16 keys each
+            float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int r = 0; r < 16; ++r) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(s[r], sl2, nm));
+                ls[r & 3] += p;
+                pb[r >> 3][r & 7] = (_Float16)p;
+            }
+            l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(s[t][f][r], sl2, nm));
-                    s[t][f][r] = p;
-                    ls += p;
-                }
-            l[f] += fa_sum_rows(ls);
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < ND; ++j)
+                    o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
         }
+        tile_wait();
+    }
 
-        // O^T += V^T P^T over two 32-key steps; k-slot 8*lg + e holds key
-        // 32*ks + 4*lg + e (e < 4) or 32*ks + 16 + 4*lg + e - 4 (e >= 4)
+    if constexpr (KS > 1) {
+        // merge the KS key shares of a query in wavefront order: (m, l, O) by
+        // LDS (the tiles are done with), added by the first wavefront
+        float* const rec = reinterpret_cast<float*>(smem) + lane;
+        constexpr int kRec = (ND * 16 + 2) * 64;
+        if (kw > 0) {
+            float* const w = rec + wave * kRec;
+            w[0] = m;
+            w[64] = l;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            fa_h8 pb[NF];
+            for (int j = 0; j < ND; ++j)
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    pb[f][r] = (_Float16)s[2 * ks][f][r];
-                    pb[f][4 + r] = (_Float16)s[2 * ks + 1][f][r];
-                }
-#pragma unroll
-            for (int j = 0; j < HD / 16; ++j) {
-                const uint16_t* vr = &Vt[cur][(16 * j + lq) * S::VROW + 32 * ks + 4 * lg];
-                const u2v lo = *reinterpret_cast<const u2v*>(vr);
-                const u2v hi = *reinterpret_cast<const u2v*>(vr + 16);
-                const u4v av = {lo.x, lo.y, hi.x, hi.y};
-                const fa_h8 a = __builtin_bit_cast(fa_h8, av);
-#pragma unroll
-                for (int f = 0; f < NF; ++f) o[j][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb[f], o[j][f], 0, 0, 0);
-            }
+                for (int r = 0; r < 16; ++r) w[(2 + 16 * j + r) * 64] = o[j][r];
         }
-        if (kb + 1 < nkb) lstore(cur ^ 1);
         __syncthreads();
-    }
-
-    // out[row][head][16j + 4*lg .. +4]: four consecutive d per fragment tile
+        if (kw > 0) return;
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const int row = row0 + 16 * (f / GB) + lq;
-        if (row >= L) continue;
-        const float inv = 1.0f / l[f];
-        uint16_t* orow = out + (int64_t)row * qstride + (int64_t)(h0 + f % GB) * HD + 4 * lg;
+        for (int i = 1; i < KS; ++i) {
+            const float* const w = rec + (wave + i) * kRec;
+            const float mo = w[0], mnew = fmaxf(m, mo);
+            const float a = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);
+            const float bsc = mo == mnew ? 1.f : __builtin_amdgcn_exp2f(mo - mnew);
+            m = mnew;
+            l = l * a + w[64] * bsc;
 #pragma unroll
-        for (int j = 0; j < HD / 16; ++j) {
-            u2v w;
-            w.x = (uint32_t)f2h(o[j][f][0] * inv) | ((uint32_t)f2h(o[j][f][1] * inv) << 16);
-            w.y = (uint32_t)f2h(o[j][f][2] * inv) | ((uint32_t)f2h(o[j][f][3] * inv) << 16);
-            *reinterpret_cast<u2v*>(orow + 16 * j) = w;
+            for (int j = 0; j < ND; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[j][r] = o[j][r] * a + w[(2 + 16 * j + r) * 64] * bsc;
         }
     }
+    l += __shfl_xor(l, 32);
+    if (row >= L) return;
+    if (sp > 1) {
+        // this part's record (O, m in natural units, l); attn_combine adds them
+        float* const rec = recs + (((int64_t)row * n_q + head) * sp + part) * (HD + 2);
+#pragma unroll
+        for (int j = 0; j < ND; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) rec[32 * j + 8 * (r >> 2) + 4 * lh + (r & 3)] = o[j][r];
+        if (lh == 0) {
+            rec[HD] = m * 0.6931471805599453f;
+            rec[HD + 1] = l;
+        }
+        return;
+    }
+    const float inv = 1.0f / l;
+    uint16_t* const orow = out + (int64_t)row * qstride + (int64_t)head * HD + 4 * lh;
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            uint16_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = f2h(o[j][4 * r4 + e] * inv);
+            if constexpr (AL) {
+                u2v w;
+                w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+                w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+                *reinterpret_cast<u2v*>(orow + 32 * j + 8 * r4) = w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) orow[32 * j + 8 * r4 + e] = h[e];
+            }
+        }
 }
 
-template <int HD, int GB, int R>
+template <int HD, int KS, bool AL = true>
 int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
-              int bidir, uint16_t* out, hipStream_t st) {
-    const int ntile = (L + 64 * R - 1) / (64 * R);
-    const int ny = n_kv * ((n_q / n_kv) / GB);
-    if (ny > 65535) return fail(BX_EINVAL, "attention: too many heads");
-    fa_kernel<HD, GB, R><<<dim3((unsigned)ntile, (unsigned)ny), 256, 0, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv,
-                                                                              bidir, out);
-    return launch_check("attention (mfma)");
+              int bidir, int gb, int sp, float* recs, uint16_t* out, hipStream_t st) {
+    using S = FaShape<HD, KS>;
+    const int rows = 32 * (4 / KS / gb);
+    const int64_t blocks = (int64_t)((L + rows - 1) / rows) * n_kv * (n_q / n_kv / gb) * sp;
+    if (blocks > (1 << 30) || n_kv > 65535) return fail(BX_EINVAL, "attention: too many heads");
+    const int cus = num_cus();
+    const int mirror = !bidir && sp == 1 && blocks > cus && blocks <= 2 * cus ? cus : (int)blocks;
+    const void* fn = reinterpret_cast<const void*>(&fa_kernel<HD, KS, AL>);
+    if (S::kLds > 64 * 1024)
+        if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds),
+                               "attention: LDS attribute"))
+            return rc;
+    fa_kernel<HD, KS, AL><<<dim3((unsigned)blocks), kFaThreads, S::kLds, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir,
+                                                                         gb, mirror, sp, recs, out);
+    if (int rc = launch_check("attention (mfma)")) return rc;
+    return sp > 1 ? attn_combine(recs, n_q, L, HD, sp, out, st) : BX_OK;
 }
 
-// Fragments per wavefront: 2 for head_dim 128 (two blocks per CU fit in the
-// register file, so one block's softmax runs under the other's MFMAs), 4 for
-// head_dim 64.  Heads per block: the largest of those, 2, 1 dividing the
-// group; the rest are 16-row fragments, halved while the grid would leave
-// CUs idle.
+// Key shares per workgroup (KS) and heads sharing a tile (gb), from the number
+// of (32 rows, head) fragments against the CUs: one fragment per wavefront
+// where they fill two workgroups per CU (2048 causal rows, 32 heads: KS 1 52
+// us, KS 2 55), two wavefronts a fragment below that (2000 rows, 16 heads: KS
+// 2 31.5 us, KS 1 42.6, KS 4 51), four where they leave CUs idle and the walk
+// over the keys is what takes the time (500 rows bidirectional, 16 heads: KS 4
+// 10.2 us, KS 2 11.5, KS 1 15.3).  Fewer fragments still over long caches:
+// `sp` workgroups share the keys, as many as the caller's workspace has
+// records for, and a second launch merges them (64 rows after 2000 keys, 16
+// heads: 13 us, one workgroup to all keys 21.9).
 template <int HD>
 int fa_dispatch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
-                int bidir, uint16_t* out, hipStream_t st) {
-    const int G = n_q / n_kv;
-    const int nf = HD == 128 ? 2 : 4;
-    int gb = (G % 4 == 0 && nf == 4) ? 4 : G % 2 == 0 ? 2 : 1;
-    auto blocks = [&](int r, int b) { return (int64_t)((L + 64 * r - 1) / (64 * r)) * n_kv * (G / b); };
-    int r = nf / gb;
-    while (r > 1 && blocks(r, gb) < num_cus()) r /= 2;
-    while (gb > 1 && blocks(r, gb) < num_cus()) gb /= 2;  // fewer heads per block: more blocks
-    if (gb == 4) return fa_launch<HD, 4, 1>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
-    if (gb == 2) {
-        if (r == 2) return fa_launch<HD, 2, 2>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
-        return fa_launch<HD, 2, 1>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
+                int bidir, void* ws, uint16_t* out, hipStream_t st) {
+    const int G = n_q / n_kv, cus = num_cus();
+    const int64_t frags = (int64_t)((L + 31) / 32) * n_q;
+    float* const recs = static_cast<float*>(ws);
+    if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(Kc) | reinterpret_cast<uintptr_t>(Vc)) & 15) ||
+        (reinterpret_cast<uintptr_t>(out) & 7))
+        return fa_launch<HD, 2, false>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, 1, recs, out, st);
+    if (frags <= cus && valid_len > 256) {
+        const int tiles = (valid_len + 127) / 128, room = attn_ws_splits(L, valid_len);
+        int sp = (int)std::min<int64_t>({cus / frags, room, tiles / 2});
+        // a tile takes 1.1 us, the second launch about 4
+        if (sp < 2 || (tiles - tiles / sp) * 1.1 < 4.5) sp = 1;
+        return fa_launch<HD, 4>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, sp, recs, out, st);
     }
-    if (r == 4) return fa_launch<HD, 1, 4>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
-    if (r == 2) return fa_launch<HD, 1, 2>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
-    return fa_launch<HD, 1, 1>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
+    if (frags <= 4 * cus) {
+        const int gb = G % 2 == 0 && frags > 2 * cus ? 2 : 1;
+        return fa_launch<HD, 2>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
+    }
+    const int gb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+    return fa_launch<HD, 1>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
 }
 
 }  // namespace
@@ -303,9 +385,9 @@ bool attn_mfma_supported(int L, int hd, float softcap, int window, const float* 
 }
 
 int attn_mfma(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
-              int hd, int bidir, uint16_t* out, hipStream_t st) {
-    if (hd == 128) return fa_dispatch<128>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
-    return fa_dispatch<64>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
+              int hd, int bidir, void* ws, uint16_t* out, hipStream_t st) {
+    if (hd == 128) return fa_dispatch<128>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, ws, out, st);
+    return fa_dispatch<64>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, ws, out, st);
 }
 
 }  // namespace bx
