@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void qk_rope_kv_rows_kernel(
 // the probabilities broadcast by readlane and EPL head dims per lane.  The key
 // parts of a head are merged in LDS; the (o, m, l) record of each (split,
 // head) goes out by device-scope stores, and the workgroup of a (row, group)
-// that finishes last merges its S records in split order (the result does not
+// that finishes last merges its T records in split order (the result does not
 // depend on arrival order), writes the FP16 output and returns the counter to
 // zero.
 template <int HD>
@@ -208,7 +208,7 @@ struct BatchAttnArgs {
     uint16_t* Kc;
     uint16_t* Vc;
     int64_t cache_rows;
-    int n_q, n_kv, S, kps, P, HPW;
+    int n_q, n_kv, S, P, HPW, max_len;
     float* recs;       // (row, group) x S x G records of HD + 2 floats
     uint64_t* cnt;     // rows x n_kv counter words (tagged_arrive), zero between launches
     uint32_t tag;      // this launch's tag (nonzero)
@@ -236,10 +236,18 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
     uint16_t* kn = qs + 8 * HD;        // the new key row
     uint16_t* vn = kn + HD;            // the new value row
     const int s = blockIdx.x, g = blockIdx.y, r = blockIdx.z;
-    const int G = a.n_q / a.n_kv, P = a.P, HPW = a.HPW, T = a.S;
+    const int G = a.n_q / a.n_kv, P = a.P, HPW = a.HPW;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int len = a.lens[r], pnew = len - 1;
-    const int kb = s * a.kps, ke = min(len, kb + a.kps);
+    // the row's own split: its keys in units of 16 over at most S workgroups,
+    // at least 64 keys each; the workgroups past the last key leave
+    const int n = max(0, min(len, a.max_len));
+    const unsigned units = ((unsigned)n + 15) >> 4;
+    const unsigned ku = max(4u, (units + (unsigned)a.S - 1) / (unsigned)a.S);
+    const int kps = 16 * (int)ku;
+    const int kb = s * kps, ke = min(n, kb + kps);
+    if (s > 0 && kb >= n) return;   // uniform over the workgroup
+    const int T = max(1, (int)((units + ku - 1) / ku));
     const bool has_cur = kb <= pnew && pnew < ke;
     const int64_t kvd = (int64_t)a.n_kv * HD;
     const int64_t row0 = a.base[r];
@@ -286,9 +294,9 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
 #pragma unroll
         for (int i = 0; i < EPL; ++i) vin[i] = vs[lane + 64 * i];
     }
-    // the first tile lands while the prologue runs; an empty split copies a
-    // row of its sequence it does not read, so every wavefront issues the
-    // same copies (the waits for the prologue's loads then count exactly)
+    // the first tile lands while the prologue runs; the split of a row without
+    // a key copies a row it does not read, so every wavefront issues the same
+    // copies (the waits for the prologue's loads then count exactly)
     copy_tile(0, max(0, min(kb, len - 1)), max(1, min(TK, ke - kb)));
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -420,7 +428,7 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
             }
         }
     }
-    // an empty split left its one tile copy in flight: it lands before the
+    // a row without a key left its one tile copy in flight: it lands before the
     // merge area (the tile buffers) is written
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();   // all waves are done with the tiles (the merge area reuses them)
@@ -467,7 +475,7 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
             }
         }
     }
-    float* grp = a.recs + ((int64_t)r * a.n_kv + g) * (int64_t)T * G * rec;
+    float* grp = a.recs + ((int64_t)r * a.n_kv + g) * (int64_t)a.S * G * rec;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(grp, 0, 0x7fffffff, 0x00020000);
     if (part == 0) {
 #pragma unroll
@@ -492,11 +500,11 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
     // the split's arrival count (tagged_arrive: a word left by a launch that
     // did not finish is not counted; the last arrival clears the word)
     uint64_t* cn = a.cnt + (int64_t)r * a.n_kv + g;
-    if (threadIdx.x == 0) last = tagged_arrive(cn, a.tag) == (uint32_t)a.S ? 1u : 0u;
+    if (threadIdx.x == 0) last = tagged_arrive(cn, a.tag) == (uint32_t)T ? 1u : 0u;
     __syncthreads();
     if (!last) return;
 
-    // ---- merge of the group's S records per head, in split order: m and l of
+    // ---- merge of the group's T records per head, in split order: m and l of
     // every record in one pass (lane t <-> record t), the weights broadcast by
     // readlane, the o rows requested sixteen records at a time
     for (int h = wave; h < G; h += 4) {
@@ -554,21 +562,28 @@ __global__ __launch_bounds__(256) void batch_attn_kernel(BatchAttnArgs a) {
     if (threadIdx.x == 0) __hip_atomic_store(cn, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Split plan of the batched attention: about two workgroups per CU over all
-// (row, group) pairs, at least 64 keys a split; P key parts per tile and HPW
-// heads per wavefront from the group size G (four wavefronts).
+// Split plan of the batched attention: S, the most splits of a row, gives
+// about two workgroups per CU over all (row, group) pairs; a row takes as many
+// of them as it has 64 keys, of equal size (from its length, on the device).
+// Sharing max_len out instead (the capacity of the slots in a decoder's step)
+// left most workgroups without keys: 16 rows of 750 to 1500 keys, 16 / 8
+// heads, 25.4 -> 22.4 us at a capacity of 1564 and 58.5 -> 22.7 us at 9564; one
+// row of 3000 at 23064 25.4 -> 14.8 us.  More workgroups than two a CU of
+// about equal size over all rows: 25.4 us at 2, 29.5 at 4, 33.8 at 6 (each has
+// a prologue and a record to merge; two fit a CU at a time).  What bounds it
+// now are the LDS reads of keys and q for the dot products.
+// P key parts per tile and HPW heads per wavefront from the group size G (four
+// wavefronts).
 struct BaPlan {
-    int S, kps, P, HPW;
+    int S, P, HPW;
 };
 inline BaPlan ba_plan(int rows, int n_q, int n_kv, int max_len) {
     BaPlan p;
     const int G = n_q / n_kv;
     p.P = G >= 4 ? 1 : 4 / G;
     p.HPW = G > 4 ? (G + 3) / 4 : 1;
-    int S = (2 * num_cus()) / max(1, rows * n_kv);
-    S = max(1, min(min(S, (max_len + 63) / 64), 256));   // the merge takes at most 256 records
-    p.kps = ((max_len + S - 1) / S + 15) / 16 * 16;
-    p.S = (max_len + p.kps - 1) / p.kps;
+    const int S = (2 * num_cus()) / max(1, rows * n_kv);
+    p.S = max(1, min(min(S, (max_len + 63) / 64), 256));   // the merge takes at most 256 records
     return p;
 }
 inline size_t ba_lds_bytes(int) { return (size_t)4 * 8192 * 2; }
@@ -630,7 +645,7 @@ int bx_batch_attention_f16(const uint16_t* q, const uint16_t* k, const uint16_t*
     a.lens = lens_dev; a.base = base_rows_dev;
     a.cos_t = cos_tab; a.sin_t = sin_tab; a.tab_rows = tab_rows;
     a.Kc = Kc; a.Vc = Vc; a.cache_rows = cache_rows;
-    a.n_q = n_q; a.n_kv = n_kv; a.S = p.S; a.kps = p.kps; a.P = p.P; a.HPW = p.HPW;
+    a.n_q = n_q; a.n_kv = n_kv; a.S = p.S; a.max_len = max_len; a.P = p.P; a.HPW = p.HPW;
     a.cnt = static_cast<uint64_t*>(workspace);
     a.tag = next_launch_tag();
     a.recs = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + cnt);

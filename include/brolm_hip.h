@@ -218,7 +218,9 @@ int bx_kv_append_rows_f16(const uint16_t* k, const uint16_t* v, int rows, int co
  * rows base_rows_dev[r] .. + lens_dev[r] - 1): the q / k head RMSNorm and RoPE
  * of bx_qk_rope_kv_rows_f16 (same bits), the new k / v rows written to the
  * cache, split attention over the row's keys and the merge of the splits ->
- * out (rows, n_q*hd) FP16.  q, k, v: the raw projections.  workspace:
+ * out (rows, n_q*hd) FP16.  max_len >= every lens_dev[r] sizes the grid and the
+ * workspace; a row is split by its own length.  q, k, v: the raw projections.
+ * workspace:
  * bx_batch_attention_workspace_bytes(rows, ...) bytes, zeroed once before its
  * first use (the kernel leaves its counters at zero; a counter left by a
  * launch that did not complete carries that launch's tag and is ignored);

@@ -248,6 +248,73 @@ def test_qk_rope_kv_rows_equals_separate_ops(hd, norm):
     assert np.array_equal(host(Kf).reshape(cap, width)[untouched], fill[untouched])
 
 
+@pytest.mark.parametrize("hd,n_q,n_kv,max_len,lens", [
+    # many ragged rows, rows without a key among them
+    (128, 4, 2, 400, [(37 * i) % 401 for i in range(70)]),
+    (64, 2, 2, 70, [64, 65, 1, 63, 0, 70] * 11 + [16]),
+    # capacity far above the contexts; one row that holds nearly all keys
+    (128, 16, 2, 30000, [17, 90, 3, 48]),
+    (128, 4, 1, 9000, [5, 9000, 1, 80]),
+    # the most splits a row can have (256), just below and at a split more keys each
+    (64, 2, 1, 40000, [20480]),
+    (64, 2, 1, 40000, [20481]),
+])
+def test_batch_attention_splits(hd, n_q, n_kv, max_len, lens):
+    """Each row's keys shared out to workgroups by its own length, whatever
+    max_len: output against a float64 softmax (the roped q is the kernel's own
+    FP16 value, the sums FP32; what is left is the FP16 rounding of outputs
+    below 4, 2^-10, and FP32 scores to 2^-10 of relative weight: atol 3e-3),
+    rows without a key give zeros, the cache rows are those of the separate
+    q / k stage, and a second launch gives the same bits."""
+    from gpu_util import call, dev, f16_dev, f16_host, host, ptr, stream, torch
+    import ctypes as C
+    import brolm_amd._native as nat
+    print(f"[batch] splits hd={hd} n_q={n_q} n_kv={n_kv} max_len={max_len} rows={len(lens)}", flush=True)
+    rng = np.random.default_rng(hd + max_len)
+    M, width = len(lens), n_kv * hd
+    lens_a = np.array(lens, np.int32)
+    base = np.concatenate([[0], np.cumsum(lens_a[:-1])]).astype(np.int64)
+    total = int(lens_a.sum())
+    q, k, v = (rng.standard_normal((M, w)) for w in (n_q * hd, width, width))
+    cache_k = rng.standard_normal((total, width)).astype(np.float16)
+    cache_v = rng.standard_normal((total, width)).astype(np.float16)
+    cos_t, sin_t = (np.empty((max_len, hd // 2), np.float32) for _ in range(2))
+    nat.hip().bx_rope_table_host(cos_t.ctypes.data_as(nat.P_f32), sin_t.ctypes.data_as(nat.P_f32), max_len, hd, 1e6)
+    cs, sn = dev(cos_t), dev(sin_t)
+    qd, kd, vd, qs = f16_dev(q), f16_dev(k), f16_dev(v), f16_dev(q)
+    pos, lens_d, base_d = dev(lens_a - 1), dev(lens_a), dev(base)
+    dst = dev(np.where(lens_a > 0, base + lens_a - 1, -1))
+    Ks, Vs = dev(cache_k.view(np.uint16)), dev(cache_v.view(np.uint16))
+    call("bx_qk_rope_kv_rows_f16", ptr(qs), ptr(kd), ptr(vd), M, hd, n_q, n_kv, None, None, C.c_float(1e-6), ptr(pos),
+         ptr(cs), ptr(sn), max_len, ptr(dst), ptr(Ks), ptr(Vs), total, ptr(qs), stream())
+    Kf, Vf = dev(cache_k.view(np.uint16)), dev(cache_v.view(np.uint16))
+    ws = torch().zeros(nat.hip().bx_batch_attention_workspace_bytes(M, n_q, n_kv, hd, max_len), dtype=torch().uint8,
+                       device="cuda")
+    outs = []
+    for _ in range(2):
+        out = torch().full((M * n_q * hd,), 0x7e00, dtype=torch().int16, device="cuda")
+        call("bx_batch_attention_f16", ptr(qd), ptr(kd), ptr(vd), M, hd, n_q, n_kv, None, None, C.c_float(1e-6),
+             ptr(lens_d), ptr(base_d), max_len, ptr(cs), ptr(sn), max_len, ptr(Kf), ptr(Vf), total, ptr(out), ptr(ws),
+             stream())
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1])
+    assert np.array_equal(host(Kf), host(Ks)) and np.array_equal(host(Vf), host(Vs))
+    Kh = host(Ks).view(np.float16).reshape(total, width).astype(np.float64)
+    Vh = host(Vs).view(np.float16).reshape(total, width).astype(np.float64)
+    qr = f16_host(qs).reshape(M, n_q, hd).astype(np.float64)
+    got = outs[0].view(np.float16).astype(np.float64).reshape(M, n_q, hd)
+    for r in range(M):
+        if lens[r] == 0:
+            assert not got[r].any()
+            continue
+        keys = slice(base[r], base[r] + lens[r])
+        for h in range(n_q):
+            g = slice(h // (n_q // n_kv) * hd, (h // (n_q // n_kv) + 1) * hd)
+            sc = Kh[keys, g] @ qr[r, h] / np.sqrt(hd)
+            w = np.exp(sc - sc.max())
+            np.testing.assert_allclose(got[r, h], (w / w.sum()) @ Vh[keys, g], atol=3e-3, err_msg=f"row {r} head {h}")
+
+
 @pytest.mark.parametrize("hd,n_q,n_kv,norm,cap", [(128, 8, 4, True, 300), (64, 8, 2, False, 200),
                                                   (256, 2, 2, True, 150), (128, 16, 2, True, 700)])
 def test_batch_attention_fused(hd, n_q, n_kv, norm, cap):
