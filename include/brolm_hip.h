@@ -220,9 +220,8 @@ int bx_kv_append_rows_f16(const uint16_t* k, const uint16_t* v, int rows, int co
  * cache, split attention over the row's keys and the merge of the splits ->
  * out (rows, n_q*hd) FP16.  max_len >= every lens_dev[r] sizes the grid and the
  * workspace; a row is split by its own length.  q, k, v: the raw projections.
- * workspace:
- * bx_batch_attention_workspace_bytes(rows, ...) bytes, zeroed once before its
- * first use (the kernel leaves its counters at zero; a counter left by a
+ * workspace: bx_batch_attention_workspace_bytes(rows, ...) bytes, zeroed once
+ * before its first use (the kernel leaves its counters at zero; a counter left by a
  * launch that did not complete carries that launch's tag and is ignored);
  * calls sharing one workspace must not overlap.  hd: 64, 128 or 256; n_q / n_kv <= 8. */
 size_t bx_batch_attention_workspace_bytes(int rows, int n_q, int n_kv, int hd, int max_len);
