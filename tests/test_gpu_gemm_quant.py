@@ -65,6 +65,31 @@ def test_quant_tiles_vs_oracle(t, M, N, K):
 
 
 @pytest.mark.parametrize("t", QTYPES)
+@pytest.mark.parametrize("M", [37, 512])
+def test_quant_tiles_multiply_the_dequantized_weights(t, M):
+    """Rows that pick one element of K each return the weights themselves: the
+    bits of bx_dequant_to_f16, also of weights near zero (blocks whose scale
+    times code all but cancels the minimum among them)."""
+    print(f"[quant weights] t={t} M={M}", flush=True)
+    N, K = 300, 512
+    rng = np.random.default_rng(60 + t)
+    raw = bytearray(sb.random_matrix(rng, t, N, K)[0])
+    if t == 12:   # d and dmin such that d * sc * q passes close to dmin * m
+        blocks = np.frombuffer(raw, np.uint8).reshape(-1, 144)
+        blocks[::2, 0:4] = np.array([0.0101, 0.0477], np.float16).view(np.uint8)
+    car = carrier(t, bytes(raw), N, K)
+    W = torch().empty(N * K, dtype=torch().int16, device="cuda")
+    call("bx_dequant_to_f16", t, ptr(car), ptr(W), N, K, stream())
+    W = f16_host(W).reshape(N, K)
+    for k0 in range(0, K, M):
+        X = np.zeros((M, K), np.float32)
+        n = min(M, K - k0)
+        X[np.arange(n), k0 + np.arange(n)] = 1
+        got = _linear(t, car, X, N)
+        assert np.array_equal(got[:n], W[:, k0:k0 + n].T), int((got[:n] != W[:, k0:k0 + n].T).sum())
+
+
+@pytest.mark.parametrize("t", QTYPES)
 def test_quant_tiles_misaligned_x_takes_the_general_kernel(t):
     """Rows that do not start on 16 bytes: the copies of 16 bytes do not take
     them; the result stays."""
