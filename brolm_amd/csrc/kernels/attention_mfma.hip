@@ -64,21 +64,21 @@ struct FaShape {
     }
 };
 
-// Eight halves at any 2-byte address.
-__device__ __forceinline__ fa_h8 fa_load8(const uint16_t* p) {
-    uint16_t v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = p[e];
-    return __builtin_bit_cast(fa_h8, v);
-}
+// Eight and four halves at any 2-byte address (one global access of 16 and 8
+// bytes: the target's unaligned access mode).
+typedef u4v __attribute__((aligned(2))) fa_any16;
+typedef u2v __attribute__((aligned(2))) fa_any8;
 
 // The larger of a query's two lanes (l and l ^ 32), in both.
 __device__ __forceinline__ float fa_pair_max(float v) { return fmaxf(v, __shfl_xor(v, 32)); }
 
-// AL: the operands are 16-byte aligned (out: 8); otherwise tiles go through
-// registers in 2-byte loads, and so do q and out.
+// AL: K and V are 16-byte aligned.  LDS-DMA takes no others; their tiles go
+// through registers, loaded before a tile's arithmetic and stored after it
+// (2048 rows of 32 / 8 heads of 128, every key visible: @@A us aligned, @@B not;
+// in 2-byte loads waited for at once it was 203).  KS = 4 holds one workgroup a
+// CU by its LDS, so its 64 registers in flight have room.
 template <int HD, int KS, bool AL>
-__global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
+__global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
                                                           const uint16_t* __restrict__ Vc, int L, int valid_len,
                                                           int n_q, int n_kv, int bidir, int gb, int mirror, int nsp,
                                                           float* __restrict__ recs, uint16_t* __restrict__ out) {
@@ -118,6 +118,7 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
     const unsigned char* const kb0 = reinterpret_cast<const unsigned char*>(Kc + (int64_t)g * HD);
     const unsigned char* const vb0 = reinterpret_cast<const unsigned char*>(Vc + (int64_t)g * HD);
     const int drow = lane / S::CH, dch = lane % S::CH;
+    u4v kreg[AL ? 1 : S::P], vreg[AL ? 1 : S::P];   // the next tile, on its way to LDS
     auto issue = [&](int kb, int buf) {
         const int k0 = kb * S::TK, left = valid_len - 1 - k0;   // keys past the end repeat the last one
         const int64_t base = (int64_t)k0 * kvstride * 2;
@@ -130,9 +131,18 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
                 dma16(off, kb0 + base, dst + j * 1024);
                 dma16(off, vb0 + base, dst + S::kTile + j * 1024);
             } else {
+                kreg[j] = *reinterpret_cast<const fa_any16*>(kb0 + base + off);
+                vreg[j] = *reinterpret_cast<const fa_any16*>(vb0 + base + off);
+            }
+        }
+    };
+    auto land = [&](int buf) {   // the tile issued last, where no copy brings it
+        if constexpr (!AL) {
+#pragma unroll
+            for (int j = 0; j < S::P; ++j) {
                 unsigned char* const d = smem + buf * S::kBuf + (wave * S::P + j) * 1024 + lane * 16;
-                *reinterpret_cast<fa_h8*>(d) = fa_load8(reinterpret_cast<const uint16_t*>(kb0 + base + off));
-                *reinterpret_cast<fa_h8*>(d + S::kTile) = fa_load8(reinterpret_cast<const uint16_t*>(vb0 + base + off));
+                *reinterpret_cast<u4v*>(d) = kreg[j];
+                *reinterpret_cast<u4v*>(d + S::kTile) = vreg[j];
             }
         }
     };
@@ -150,7 +160,7 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
         const uint16_t* qrow = q + (int64_t)min(row, L - 1) * qstride + (int64_t)head * HD + 8 * lh;
 #pragma unroll
         for (int s = 0; s < HD / 16; ++s)
-            qf[s] = AL ? *reinterpret_cast<const fa_h8*>(qrow + 16 * s) : fa_load8(qrow + 16 * s);
+            qf[s] = __builtin_bit_cast(fa_h8, (u4v)*reinterpret_cast<const fa_any16*>(qrow + 16 * s));
         // waited for here: left to their first use, inside the loop, the wait
         // would also cover the tile copies just issued there, every iteration
 #pragma unroll
@@ -173,7 +183,10 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
     const int vkey = kw * S::WK + 4 * lh + (ti >> 2), vcol = 2 * tg + ((ti & 3) >> 1), vb8 = (ti & 1) * 8;
 
     const int kb_first = (int)((int64_t)nkb * part / sp), kb_end = (int)((int64_t)nkb * (part + 1) / sp);
-    if (kb_first < kb_end) issue(kb_first, 0);
+    if (kb_first < kb_end) {
+        issue(kb_first, 0);
+        land(0);
+    }
     tile_wait();
     for (int kb = kb_first; kb < kb_end; ++kb) {
         const int cur = (kb - kb_first) & 1;
@@ -255,6 +268,7 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
                 for (int j = 0; j < ND; ++j)
                     o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
         }
+        if (kb + 1 < kb_end) land(cur ^ 1);
         tile_wait();
     }
 
@@ -312,19 +326,14 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_kernel(const uint16_t* __res
             uint16_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) h[e] = f2h(o[j][4 * r4 + e] * inv);
-            if constexpr (AL) {
-                u2v w;
-                w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
-                w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-                *reinterpret_cast<u2v*>(orow + 32 * j + 8 * r4) = w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) orow[32 * j + 8 * r4 + e] = h[e];
-            }
+            u2v w;
+            w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+            w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+            *reinterpret_cast<fa_any8*>(orow + 32 * j + 8 * r4) = w;
         }
 }
 
-template <int HD, int KS, bool AL = true>
+template <int HD, int KS, bool AL>
 int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
               int bidir, int gb, int sp, float* recs, uint16_t* out, hipStream_t st) {
     using S = FaShape<HD, KS>;
@@ -354,28 +363,25 @@ int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, 
 // `sp` workgroups share the keys, as many as the caller's workspace has
 // records for, and a second launch merges them (64 rows after 2000 keys, 16
 // heads: 13 us, one workgroup to all keys 21.9).
-template <int HD>
+template <int HD, bool AL>
 int fa_dispatch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
                 int bidir, void* ws, uint16_t* out, hipStream_t st) {
     const int G = n_q / n_kv, cus = num_cus();
     const int64_t frags = (int64_t)((L + 31) / 32) * n_q;
     float* const recs = static_cast<float*>(ws);
-    if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(Kc) | reinterpret_cast<uintptr_t>(Vc)) & 15) ||
-        (reinterpret_cast<uintptr_t>(out) & 7))
-        return fa_launch<HD, 2, false>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, 1, recs, out, st);
     if (frags <= cus && valid_len > 256) {
         const int tiles = (valid_len + 127) / 128, room = attn_ws_splits(L, valid_len);
         int sp = (int)std::min<int64_t>({cus / frags, room, tiles / 2});
         // a tile takes 1.1 us, the second launch about 4
         if (sp < 2 || (tiles - tiles / sp) * 1.1 < 4.5) sp = 1;
-        return fa_launch<HD, 4>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, sp, recs, out, st);
+        return fa_launch<HD, 4, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, sp, recs, out, st);
     }
     if (frags <= 4 * cus) {
         const int gb = G % 2 == 0 && frags > 2 * cus ? 2 : 1;
-        return fa_launch<HD, 2>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
+        return fa_launch<HD, 2, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
     }
     const int gb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-    return fa_launch<HD, 1>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
+    return fa_launch<HD, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
 }
 
 }  // namespace
@@ -386,8 +392,10 @@ bool attn_mfma_supported(int L, int hd, float softcap, int window, const float* 
 
 int attn_mfma(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
               int hd, int bidir, void* ws, uint16_t* out, hipStream_t st) {
-    if (hd == 128) return fa_dispatch<128>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, ws, out, st);
-    return fa_dispatch<64>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, ws, out, st);
+    const bool al = ((reinterpret_cast<uintptr_t>(Kc) | reinterpret_cast<uintptr_t>(Vc)) & 15) == 0;
+    const auto run = hd == 128 ? (al ? fa_dispatch<128, true> : fa_dispatch<128, false>)
+                               : (al ? fa_dispatch<64, true> : fa_dispatch<64, false>);
+    return run(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, ws, out, st);
 }
 
 }  // namespace bx
