@@ -10,11 +10,15 @@
 // rows over different keys of a tile, merged at the end (small problems, where
 // the serial walk over the keys is what takes the time).  Keys and values come
 // in tiles by LDS-DMA, double buffered, rows as stored, 16-byte chunks
-// XOR-swizzled by the key.  Per 32 keys, on v_mfma_f32_32x32x16_f16:
-//   S^T = K Q^T     (a lane holds 16 of the 32 keys of its query)
+// XOR-swizzled by the key.  Per step of NK fragments of 32 keys (two where a
+// wavefront has all 64 of a tile, else one), on v_mfma_f32_32x32x16_f16:
+//   S^T = K Q^T     (a lane holds 16 of a fragment's 32 keys of its query)
 //   online softmax  (base-2 exponent, running max per query in FP32, moved only
-//                    when some tile max exceeds it by more than 2^8; a lane
-//                    sums its own keys, the halves of a query add at the end)
+//                    when some step's max exceeds it by more than 2^8; a lane
+//                    sums its own keys, the halves of a query add at the end).
+//                    The max of 64 keys and not of 32: the weight of the
+//                    largest key so far is exactly 1 in FP16 more often, which
+//                    is 0.8 % of the error of 2048 causal rows
 //   O^T += V^T P^T  (P to FP16 in registers: the S^T layout is the B operand's
 //                    with the keys of a k-slot group in a fixed order; V^T
 //                    comes out of the row-major tile by transposing LDS reads,
@@ -74,8 +78,8 @@ __device__ __forceinline__ float fa_pair_max(float v) { return fmaxf(v, __shfl_x
 
 // AL: K and V are 16-byte aligned.  LDS-DMA takes no others; their tiles go
 // through registers, loaded before a tile's arithmetic and stored after it
-// (2048 rows of 32 / 8 heads of 128, every key visible: @@A us aligned, @@B not;
-// in 2-byte loads waited for at once it was 203).  KS = 4 holds one workgroup a
+// (2048 rows of 32 / 8 heads of 128, every key visible: 77 us aligned, 90 on 8
+// bytes, 106 on 2; in 2-byte loads waited for at once 203 and 228).  KS = 4 holds one workgroup a
 // CU by its LDS, so its 64 registers in flight have room.
 template <int HD, int KS, bool AL>
 __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
@@ -193,48 +197,62 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
         if (kb + 1 < kb_end) issue(kb + 1, cur ^ 1);
         const unsigned char* const kt = smem + cur * S::kBuf;
         const unsigned char* const vt = kt + S::kTile;
+        const int key0 = kb * S::TK + kw * S::WK;
+        if (key0 <= any_see) {
+            // fragments of 32 keys some query sees
+            const bool more = NK > 1 && key0 + 32 <= any_see;
+            // S^T: lane l, register r of s[t] holds key 32 t + 8 (r / 4) + 4 lh + r % 4
+            fa_f16 s[NK];
 #pragma unroll
-        for (int t = 0; t < NK; ++t) {
-            const int key0 = kb * S::TK + kw * S::WK + 32 * t;   // 32 keys at a time
-            if (key0 > any_see) break;
-            fa_h8 kf[HD / 16];
+            for (int t = 0; t < NK; ++t) {
 #pragma unroll
-            for (int d = 0; d < HD / 16; ++d)
-                kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + t * 32 * S::RB + (((2 * d) ^ kx) << 4));
-            __builtin_amdgcn_sched_barrier(0);
-            fa_f16 s;
+                for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
+                if (t > 0 && !more) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 0.f;
+                    for (int r = 0; r < 16; ++r) s[t][r] = -INFINITY;
+                    continue;
+                }
+                fa_h8 kf[HD / 16];
 #pragma unroll
-            for (int d = 0; d < HD / 16; ++d) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[d], qf[d], s, 0, 0, 0);
+                for (int d = 0; d < HD / 16; ++d)
+                    kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + t * 32 * S::RB + (((2 * d) ^ kx) << 4));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int d = 0; d < HD / 16; ++d)
+                    s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[d], qf[d], s[t], 0, 0, 0);
+            }
             // the values are requested before the softmax that weighs them:
             // k-slot (lh, e) of V^T holds key 16 u + 4 lh + e (e < 4) or 16 u +
             // 8 + 4 lh + e - 4 (e >= 4)
             fa_h8 vf[2][ND];
+            auto values = [&](int t) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+                for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int j = 0; j < ND; ++j) {
-                    const int c = 4 * j + vcol;
-                    const int k1 = 32 * t + 16 * u + vkey, k2 = k1 + 8;
-                    const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + vb8;
-                    const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + vb8;
-                    const fa_h4 lo = __builtin_bit_cast(
-                        fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a1));
-                    const fa_h4 hi = __builtin_bit_cast(
-                        fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a2));
-                    vf[u][j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                }
+                    for (int j = 0; j < ND; ++j) {
+                        const int c = 4 * j + vcol;
+                        const int k1 = 32 * t + 16 * u + vkey, k2 = k1 + 8;
+                        const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + vb8;
+                        const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + vb8;
+                        const fa_h4 lo = __builtin_bit_cast(
+                            fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a1));
+                        const fa_h4 hi = __builtin_bit_cast(
+                            fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a2));
+                        vf[u][j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                    }
+            };
+            values(0);
             __builtin_amdgcn_sched_barrier(0);
-            // lane l, register r: key 8 (r / 4) + 4 lh + r % 4
-            if (key0 + 31 > all_see) {
+            if (key0 + S::WK - 1 > all_see) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (key0 + 8 * (r >> 2) + 4 * lh + (r & 3) > last_key) s[r] = -INFINITY;
+                for (int t = 0; t < NK; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (key0 + 32 * t + 8 * (r >> 2) + 4 * lh + (r & 3) > last_key) s[t][r] = -INFINITY;
             }
-            float mx = fmaxf(s[0], s[1]);
+            float mx = fmaxf(s[0][0], s[0][1]);
 #pragma unroll
-            for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            for (int r = 2; r < 16 * NK; ++r) mx = fmaxf(mx, s[r / 16][r % 16]);
             mx = fa_pair_max(mx) * sl2;  // the tile's max in base-2 units (sl2 > 0)
             // v_exp_f32 flushes results below 2^-126 to zero: weights that
             // small (scores 87 natural units under the row max) are zero in
@@ -253,20 +271,25 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
                 m = mnew;
             }
             const float nm = m == -INFINITY ? 0.f : -m;
-            fa_h8 pb[2];   // B operands: 16 keys each
-            float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(s[r], sl2, nm));
-                ls[r & 3] += p;
-                pb[r >> 3][r & 7] = (_Float16)p;
+            for (int t = 0; t < NK; ++t) {
+                if (t > 0 && !more) break;
+                fa_h8 pb[2];   // B operands: 16 keys each
+                float ls[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float p = __builtin_amdgcn_exp2f(fmaf(s[t][r], sl2, nm));
+                    ls[r & 3] += p;
+                    pb[r >> 3][r & 7] = (_Float16)p;
+                }
+                l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+                if (t > 0) values(t);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int j = 0; j < ND; ++j)
+                        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
             }
-            l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int j = 0; j < ND; ++j)
-                    o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
         }
         if (kb + 1 < kb_end) land(cur ^ 1);
         tile_wait();
