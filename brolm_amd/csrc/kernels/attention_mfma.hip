@@ -30,9 +30,11 @@
 // the LDS reads of both operands (16 KB, which is why one fragment of K feeds
 // 32 queries and not 16).  Measured against 16-row fragments with tiles staged
 // through registers and V transposed on its way into LDS: 2048 causal rows of
-// 32 / 8 heads of 128 100.5 -> 54.0 us (640 TFLOP/s), 500 rows bidirectional
-// of 16 heads 19.8 -> 10.4 us, 1024 rows after 1500 of 32 heads 102 -> 52 us,
-// 64 rows after 2000 of 16 heads 62 -> 13 us.
+// 32 / 8 heads of 128 100 -> 51.7 us (660 TFLOP/s), 500 rows bidirectional
+// of 16 heads 17.8 -> 9.3 us, 700 rows after 2000 of 16 heads 87 -> 36 us,
+// 64 rows after 2000 of 16 heads 62 -> 12.1 us.  Calls of up to 64 rows over 33
+// to 64 keys are the exception (64 rows of 16 heads 5.1 -> 5.6 us): a fragment
+// of 32 rows has twice the serial work of one of 16.
 #include <algorithm>
 
 #include "attention_core.h"
@@ -45,21 +47,25 @@ typedef _Float16 fa_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 fa_h4 __attribute__((ext_vector_type(4)));
 typedef short fa_s4 __attribute__((ext_vector_type(4)));
 typedef float fa_f16 __attribute__((ext_vector_type(16)));
+typedef float fa_f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kFaThreads = 256;
 
-template <int HD, int KS>
+template <int HD, int KS, int NK>
 struct FaShape {
     static constexpr int TK = KS == 4 ? 128 : 64;       // keys per tile
     static constexpr int WK = TK / KS;                  // keys per wavefront and tile
-    static constexpr int NK = WK / 32;                  // 32-key fragments per wavefront and tile
+    static constexpr int SK = 32 * NK;                  // keys per step: NK fragments of 32
+    static_assert(WK == SK || WK == 2 * SK);
     static constexpr int RB = HD * 2;                   // bytes per key row
     static constexpr int CH = HD / 8;                   // 16-byte chunks per key row
     static constexpr int RPC = 1024 / RB;               // rows per copy instruction
     static constexpr int P = TK / RPC / 4;              // copies per wavefront and tile, of K and of V
     static constexpr int kTile = TK * RB;               // bytes of a K (or V) tile
     static constexpr int kBuf = 2 * kTile;
-    static constexpr int kMerge = KS > 1 ? 4 * 64 * (HD / 32 * 16 + 2) * 4 : 0;   // end merge, FP32
+    static constexpr int QW = HD / 8 / KS;              // quads of O^T a wavefront finishes
+    static constexpr int kRec = (HD / 8 - QW + 1) * 64; // 16-byte words of a wavefront's end-merge record
+    static constexpr int kMerge = KS > 1 ? 4 * kRec * 16 : 0;
     static constexpr int kLds = 2 * kBuf > kMerge ? 2 * kBuf : kMerge;
     // chunk c of key k sits at c ^ swz(k): the 16 keys a K read covers land on
     // distinct chunks of the banks, and so do the 4 keys of a transposing read
@@ -81,13 +87,13 @@ __device__ __forceinline__ float fa_pair_max(float v) { return fmaxf(v, __shfl_x
 // (2048 rows of 32 / 8 heads of 128, every key visible: 77 us aligned, 90 on 8
 // bytes, 106 on 2; in 2-byte loads waited for at once 203 and 228).  KS = 4 holds one workgroup a
 // CU by its LDS, so its 64 registers in flight have room.
-template <int HD, int KS, bool AL>
+template <int HD, int KS, int NK, bool AL>
 __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc,
                                                           const uint16_t* __restrict__ Vc, int L, int valid_len,
                                                           int n_q, int n_kv, int bidir, int gb, int mirror, int nsp,
                                                           float* __restrict__ recs, uint16_t* __restrict__ out) {
-    using S = FaShape<HD, KS>;
-    constexpr int NK = S::NK, ND = HD / 32;
+    using S = FaShape<HD, KS, NK>;
+    constexpr int ND = HD / 32;
     extern __shared__ __align__(1024) unsigned char smem[];
 
     // block -> (row tile, head set): latest rows first (they see the most
@@ -114,7 +120,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
     const int last_key = bidir ? valid_len - 1 : min(p0 + row, valid_len - 1);
     // keys every query of the wavefront sees (its first row's)
     const int all_see = bidir ? valid_len - 1 : min(p0 + row0, valid_len - 1);
-    // keys some query of the wavefront sees
+    // keys some query of the wavefront sees; none where its rows end above it
     const int any_see = bidir ? valid_len - 1 : min(p0 + row0 + 31, valid_len - 1);
 
     // ---- copies: wavefront w takes rows RPC (w P + j) .. of a tile
@@ -197,8 +203,9 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
         if (kb + 1 < kb_end) issue(kb + 1, cur ^ 1);
         const unsigned char* const kt = smem + cur * S::kBuf;
         const unsigned char* const vt = kt + S::kTile;
-        const int key0 = kb * S::TK + kw * S::WK;
-        if (key0 <= any_see) {
+        auto step = [&](int st) {   // keys st .. st + SK - 1 of the wavefront's share
+            const int key0 = kb * S::TK + kw * S::WK + st;
+            if (key0 > any_see) return;
             // fragments of 32 keys some query sees
             const bool more = NK > 1 && key0 + 32 <= any_see;
             // S^T: lane l, register r of s[t] holds key 32 t + 8 (r / 4) + 4 lh + r % 4
@@ -215,7 +222,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
                 fa_h8 kf[HD / 16];
 #pragma unroll
                 for (int d = 0; d < HD / 16; ++d)
-                    kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + t * 32 * S::RB + (((2 * d) ^ kx) << 4));
+                    kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + (st + 32 * t) * S::RB + (((2 * d) ^ kx) << 4));
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int d = 0; d < HD / 16; ++d)
@@ -231,7 +238,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
 #pragma unroll
                     for (int j = 0; j < ND; ++j) {
                         const int c = 4 * j + vcol;
-                        const int k1 = 32 * t + 16 * u + vkey, k2 = k1 + 8;
+                        const int k1 = st + 32 * t + 16 * u + vkey, k2 = k1 + 8;
                         const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + vb8;
                         const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + vb8;
                         const fa_h4 lo = __builtin_bit_cast(
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
             };
             values(0);
             __builtin_amdgcn_sched_barrier(0);
-            if (key0 + S::WK - 1 > all_see) {
+            if (key0 + S::SK - 1 > all_see) {
 #pragma unroll
                 for (int t = 0; t < NK; ++t)
 #pragma unroll
@@ -262,7 +269,8 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
             // well inside FP16).  A query that has seen no key yet has m =
             // -inf: its first visible tile moves it, and until then every
             // weight is exp2(-inf - finite) = 0 (nm below).
-            if (__any(mx > m + 8.f)) {
+            // (Two steps of one tile: any larger max, as one step would have it.)
+            if (__any(mx > m + (S::WK > S::SK ? 0.f : 8.f))) {
                 const float mnew = fmaxf(m, mx);
                 const float alpha = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);
                 l *= alpha;
@@ -290,87 +298,123 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
                     for (int j = 0; j < ND; ++j)
                         o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
             }
-        }
+        };
+        step(0);
+        if constexpr (S::WK > S::SK) step(S::SK);
         if (kb + 1 < kb_end) land(cur ^ 1);
         tile_wait();
     }
 
-    if constexpr (KS > 1) {
-        // merge the KS key shares of a query in wavefront order: (m, l, O) by
-        // LDS (the tiles are done with), added by the first wavefront
-        float* const rec = reinterpret_cast<float*>(smem) + lane;
-        constexpr int kRec = (ND * 16 + 2) * 64;
-        if (kw > 0) {
-            float* const w = rec + wave * kRec;
-            w[0] = m;
-            w[64] = l;
+    // The KS wavefronts of a query each finish QW of the 4 ND quads of O^T (quad
+    // x = 4 j + r / 4: four head dims of the lane's query): they hand the others'
+    // quads over through LDS (the tiles are done with) and add the shares of
+    // their own in wavefront order.  Left to one wavefront, the merge and the
+    // stores were 0.9 of 5.0 us of the smallest calls.
+    constexpr int QW = S::QW;
+    fa_f4 own[QW];
+    auto quad = [&](int x) {
+        const fa_f16& f = o[x / 4];
+        return fa_f4{f[4 * (x % 4)], f[4 * (x % 4) + 1], f[4 * (x % 4) + 2], f[4 * (x % 4) + 3]};
+    };
+    if constexpr (KS == 1) {
 #pragma unroll
-            for (int j = 0; j < ND; ++j)
+        for (int x = 0; x < QW; ++x) own[x] = quad(x);
+    } else {
+        fa_f4* const recs0 = reinterpret_cast<fa_f4*>(smem) + lane;
+        fa_f4* const mine = recs0 + wave * S::kRec;
+        if (row0 < L) {
+            static_for<KS>([&](auto c) {
+                constexpr int k = decltype(c)::value;
+                if (kw == k) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) w[(2 + 16 * j + r) * 64] = o[j][r];
+                    for (int x = 0; x < 4 * ND; ++x) {
+                        if (x / QW == k) own[x % QW] = quad(x);
+                        else mine[(x < k * QW ? x : x - QW) * 64] = quad(x);
+                    }
+                }
+            });
+            mine[(4 * ND - QW) * 64] = fa_f4{m, l, 0.f, 0.f};
         }
         __syncthreads();
-        if (kw > 0) return;
+        if (row0 >= L) return;
+        float ms = 0.f, ls = 0.f;
+        fa_f4 sum[QW];
 #pragma unroll
-        for (int i = 1; i < KS; ++i) {
-            const float* const w = rec + (wave + i) * kRec;
-            const float mo = w[0], mnew = fmaxf(m, mo);
-            const float a = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);
-            const float bsc = mo == mnew ? 1.f : __builtin_amdgcn_exp2f(mo - mnew);
-            m = mnew;
-            l = l * a + w[64] * bsc;
+        for (int i = 0; i < KS; ++i) {
+            const fa_f4* const r = recs0 + (qw * KS + i) * S::kRec;
+            const fa_f4 ml = r[(4 * ND - QW) * 64];
+            fa_f4 v[QW];
 #pragma unroll
-            for (int j = 0; j < ND; ++j)
+            for (int x = 0; x < QW; ++x) {
+                v[x] = own[x];
+                if (i != kw) v[x] = r[((kw < i ? kw : kw - 1) * QW + x) * 64];
+            }
+            if (i == 0) {
+                ms = ml[0];
+                ls = ml[1];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) o[j][r] = o[j][r] * a + w[(2 + 16 * j + r) * 64] * bsc;
+                for (int x = 0; x < QW; ++x) sum[x] = v[x];
+            } else {
+                const float mnew = fmaxf(ms, ml[0]);
+                const float a = ms == mnew ? 1.f : __builtin_amdgcn_exp2f(ms - mnew);
+                const float b = ml[0] == mnew ? 1.f : __builtin_amdgcn_exp2f(ml[0] - mnew);
+                ms = mnew;
+                ls = ls * a + ml[1] * b;
+#pragma unroll
+                for (int x = 0; x < QW; ++x) sum[x] = sum[x] * a + v[x] * b;
+            }
         }
+        m = ms;
+        l = ls;
+#pragma unroll
+        for (int x = 0; x < QW; ++x) own[x] = sum[x];
     }
     l += __shfl_xor(l, 32);
     if (row >= L) return;
+    // head dim of element 0 of own quad x
+    auto dim = [&](int x) { return 8 * (kw * QW + x) + 4 * lh; };
     if (sp > 1) {
         // this part's record (O, m in natural units, l); attn_combine adds them
         float* const rec = recs + (((int64_t)row * n_q + head) * sp + part) * (HD + 2);
 #pragma unroll
-        for (int j = 0; j < ND; ++j)
+        for (int x = 0; x < QW; ++x)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) rec[32 * j + 8 * (r >> 2) + 4 * lh + (r & 3)] = o[j][r];
-        if (lh == 0) {
+            for (int e = 0; e < 4; ++e) rec[dim(x) + e] = own[x][e];
+        if (kw == 0 && lh == 0) {
             rec[HD] = m * 0.6931471805599453f;
             rec[HD + 1] = l;
         }
         return;
     }
     const float inv = 1.0f / l;
-    uint16_t* const orow = out + (int64_t)row * qstride + (int64_t)head * HD + 4 * lh;
+    uint16_t* const orow = out + (int64_t)row * qstride + (int64_t)head * HD;
 #pragma unroll
-    for (int j = 0; j < ND; ++j)
+    for (int x = 0; x < QW; ++x) {
+        uint16_t h[4];
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            uint16_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = f2h(o[j][4 * r4 + e] * inv);
-            u2v w;
-            w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
-            w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-            *reinterpret_cast<fa_any8*>(orow + 32 * j + 8 * r4) = w;
-        }
+        for (int e = 0; e < 4; ++e) h[e] = f2h(own[x][e] * inv);
+        u2v w;
+        w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+        w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+        *reinterpret_cast<fa_any8*>(orow + dim(x)) = w;
+    }
 }
 
-template <int HD, int KS, bool AL>
+template <int HD, int KS, int NK, bool AL>
 int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
               int bidir, int gb, int sp, float* recs, uint16_t* out, hipStream_t st) {
-    using S = FaShape<HD, KS>;
+    using S = FaShape<HD, KS, NK>;
     const int rows = 32 * (4 / KS / gb);
     const int64_t blocks = (int64_t)((L + rows - 1) / rows) * n_kv * (n_q / n_kv / gb) * sp;
     if (blocks > (1 << 30) || n_kv > 65535) return fail(BX_EINVAL, "attention: too many heads");
     const int cus = num_cus();
     const int mirror = !bidir && sp == 1 && blocks > cus && blocks <= 2 * cus ? cus : (int)blocks;
-    const void* fn = reinterpret_cast<const void*>(&fa_kernel<HD, KS, AL>);
+    const void* fn = reinterpret_cast<const void*>(&fa_kernel<HD, KS, NK, AL>);
     if (S::kLds > 64 * 1024)
         if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds),
                                "attention: LDS attribute"))
             return rc;
-    fa_kernel<HD, KS, AL><<<dim3((unsigned)blocks), kFaThreads, S::kLds, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir,
+    fa_kernel<HD, KS, NK, AL><<<dim3((unsigned)blocks), kFaThreads, S::kLds, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir,
                                                                          gb, mirror, sp, recs, out);
     if (int rc = launch_check("attention (mfma)")) return rc;
     return sp > 1 ? attn_combine(recs, n_q, L, HD, sp, out, st) : BX_OK;
@@ -382,29 +426,33 @@ int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, 
 // us, KS 2 55), two wavefronts a fragment below that (2000 rows, 16 heads: KS
 // 2 31.5 us, KS 1 42.6, KS 4 51), four where they leave CUs idle and the walk
 // over the keys is what takes the time (500 rows bidirectional, 16 heads: KS 4
-// 10.2 us, KS 2 11.5, KS 1 15.3).  Fewer fragments still over long caches:
+// 9.3 us, KS 2 11.5, KS 1 15.3).  Fewer fragments still over long caches:
 // `sp` workgroups share the keys, as many as the caller's workspace has
 // records for, and a second launch merges them (64 rows after 2000 keys, 16
-// heads: 13 us, one workgroup to all keys 21.9).
+// heads: 12 us, one workgroup to all keys 21.9).
 template <int HD, bool AL>
 int fa_dispatch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
                 int bidir, void* ws, uint16_t* out, hipStream_t st) {
     const int G = n_q / n_kv, cus = num_cus();
     const int64_t frags = (int64_t)((L + 31) / 32) * n_q;
     float* const recs = static_cast<float*>(ws);
+    // the smallest calls: one tile, no merge (16 heads of 128: 16 rows and keys
+    // 4.1 us, KS 2 4.8; 64 rows and keys 5.6, KS 2 5.9)
+    if (valid_len <= 64)
+        return fa_launch<HD, 1, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, 1, recs, out, st);
     if (frags <= cus && valid_len > 256) {
         const int tiles = (valid_len + 127) / 128, room = attn_ws_splits(L, valid_len);
         int sp = (int)std::min<int64_t>({cus / frags, room, tiles / 2});
         // a tile takes 1.1 us, the second launch about 4
         if (sp < 2 || (tiles - tiles / sp) * 1.1 < 4.5) sp = 1;
-        return fa_launch<HD, 4, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, sp, recs, out, st);
+        return fa_launch<HD, 4, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, sp, recs, out, st);
     }
     if (frags <= 4 * cus) {
         const int gb = G % 2 == 0 && frags > 2 * cus ? 2 : 1;
-        return fa_launch<HD, 2, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
+        return fa_launch<HD, 2, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
     }
     const int gb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-    return fa_launch<HD, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
+    return fa_launch<HD, 1, 2, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, gb, 1, recs, out, st);
 }
 
 }  // namespace
