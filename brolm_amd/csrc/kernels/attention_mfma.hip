@@ -410,10 +410,10 @@ int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, 
     const int cus = num_cus();
     const int mirror = !bidir && sp == 1 && blocks > cus && blocks <= 2 * cus ? cus : (int)blocks;
     const void* fn = reinterpret_cast<const void*>(&fa_kernel<HD, KS, NK, AL>);
-    if (S::kLds > 64 * 1024)
-        if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds),
-                               "attention: LDS attribute"))
-            return rc;
+    if constexpr (S::kLds > 64 * 1024) {
+        static std::atomic<uint64_t> allowed{0};
+        if (int rc = allow_lds(allowed, fn, S::kLds, "attention: LDS attribute")) return rc;
+    }
     fa_kernel<HD, KS, NK, AL><<<dim3((unsigned)blocks), kFaThreads, S::kLds, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir,
                                                                          gb, mirror, sp, recs, out);
     if (int rc = launch_check("attention (mfma)")) return rc;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -35,6 +36,10 @@ uint32_t next_launch_tag();
 // holds at once for kernel `fn` (registers and LDS); asked of the runtime once
 // per (kernel, threads, LDS) and cached; at least 1.
 int resident_wgs(const void* fn, int threads, size_t lds);
+// Lets kernel `fn` use `bytes` of dynamic LDS (more than 64 KB has to be allowed
+// per kernel and device).  `done`, one per kernel, holds a bit per device for
+// which it was: the runtime call costs 0.3 to 0.5 us, an eighth of a launch.
+int allow_lds(std::atomic<uint64_t>& done, const void* fn, int bytes, const char* what);
 
 // Workgroups per CU launched for the wide-row GEMVs (K above 12288), one
 // round of residents: a lane's 128+ registers and up to 80 KB of staged

@@ -235,9 +235,8 @@ int launch(TileJob job, const uint16_t* bias, const uint16_t* X, int M, int K, i
     tiles *= job.tiles_m;
     if (tiles > (1 << 30)) return fail(BX_EINVAL, "gemm: too many tiles");
     const void* fn = reinterpret_cast<const void*>(&gemm_f16_kernel<Sh>);
-    if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, Sh::kLds),
-                           "gemm f16: LDS attribute"))
-        return rc;
+    static std::atomic<uint64_t> allowed{0};
+    if (int rc = allow_lds(allowed, fn, Sh::kLds, "gemm f16: LDS attribute")) return rc;
     gemm_f16_kernel<Sh><<<dim3((unsigned)tiles), Sh::NT, Sh::kLds, st>>>(job, X, bias, M, K, epi);
     return launch_check("gemm_f16");
 }

@@ -614,9 +614,8 @@ int launch_quant(QuantJob job, const uint16_t* bias, const uint16_t* X, int M, i
     tiles *= (int64_t)job.t.tiles_m * job.S;
     if (tiles > (1 << 30)) return fail(BX_EINVAL, "gemm: too many tiles");
     const void* fn = reinterpret_cast<const void*>(&gemm_quant_kernel<FMT, FM, FN>);
-    if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, Sh::kLds),
-                           "gemm quant: LDS attribute"))
-        return rc;
+    static std::atomic<uint64_t> allowed{0};
+    if (int rc = allow_lds(allowed, fn, Sh::kLds, "gemm quant: LDS attribute")) return rc;
     gemm_quant_kernel<FMT, FM, FN><<<dim3((unsigned)tiles), kThreads, Sh::kLds, st>>>(job, X, bias, M, K, epi);
     return launch_check("gemm_quant");
 }

@@ -58,6 +58,16 @@ int resident_wgs(const void* fn, int threads, size_t lds) {
     return occ;
 }
 
+int allow_lds(std::atomic<uint64_t>& done, const void* fn, int bytes, const char* what) {
+    int dev = 0;
+    if (int rc = hip_check(hipGetDevice(&dev), what)) return rc;
+    const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;   // past 64 devices: asked every time
+    if (done.load(std::memory_order_acquire) & bit) return BX_OK;
+    if (int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes), what)) return rc;
+    done.fetch_or(bit, std::memory_order_release);
+    return BX_OK;
+}
+
 // rocprofv3 injects its tool by LD_PRELOAD of librocprofiler-sdk-tool.so and
 // names it in ROCP_TOOL_LIBRARIES.  Under that tool, a process whose kernels
 // were launched cooperatively, or through a hipGraph, has ended in a host
