@@ -17,9 +17,9 @@
 //  - gemm_kernel<FMT> (other shapes): 64x64 block tile, K step 32, 4
 //    wavefronts each a 32x32 quadrant of 16x16x16 MFMAs.
 // They serve what the LDS-DMA kernels leave: quantized weights with K a
-// multiple of 256 run gemm_quant.hip, FP16 weights with K a multiple of 64
-// gemm_f16.hip, at any M above 16 with 16-byte aligned operands
-// (gemm_quant_ok, gemm_f16_ok).
+// multiple of 256 run gemm_quant.hip (Q6_K with an even count of blocks), FP16
+// weights with K a multiple of 64 gemm_f16.hip, at any M above 16 with 16-byte
+// aligned operands (gemm_quant_ok, gemm_f16_ok).
 #include "carrier_layout.h"
 #include "gemm_job.h"
 

@@ -13,8 +13,11 @@ namespace bx {
 // runs over the members' column tiles in order.  EPI_STORE writes Y = f16(acc
 // + bias); EPI_RESID adds f16(acc) to the FP32 residual H[M, N[0]]; EPI_SWIGLU
 // computes gate (W[0]) and up (W[1]) columns of the same tile and writes Y[0] =
-// f16(f16(silu(f16(gate))) * f16(up)), the values the separate linear, silu
-// and mul kernels give.
+// f16(f16(silu(f16(gate))) * f16(up)).  EPI_RESID and EPI_SWIGLU give the bits of
+// the separate linear, add, silu and mul kernels (weights on 16-byte
+// boundaries); several members give those of their plain launches too, but for
+// quantized weights whose K slices differ there (gemm_quant.hip), where they
+// differ by the order of FP32 sums.
 enum : int { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2 };
 struct TileJob {
     const void* W[3];

@@ -564,6 +564,16 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_quant_kernel(QuantJob job, c
 // then MFMA-bound), more when every CU streams; a split adds the exchange of
 // its partials.  Example: 75 x 6144 x 2048 Q4_K takes 13.1 us as 32-row tiles,
 // 14.7 us as 96-row tiles in 4 slices, 28 us as 96 x 256 tiles.
+//
+// The slices decide the order in which an output's sums are added.  A residual
+// launch has those of the plain launch, being planned alike, and SwiGLU takes
+// those of the plain launch of gate or up: both give the bits of the separate
+// ops.  (Its own slices would be faster only for Q6_K of few columns: 128 x 3072
+// x 1024 13.8 us, 15.1 so.)  q / k / v in one launch have slices of their own:
+// those of the separate launches, which fill the chip three times over, cost up
+// to twice the time (200 rows of 2048 + 1024 + 1024 columns, K = 2048, Q4_K 12.9
+// us against 28.8), so a group's sums may differ from the plain launches' in the
+// last bits of FP32.
 struct QPlan {
     int fm, fn, S;
 };
@@ -572,24 +582,31 @@ QPlan quant_plan(const TileJob& job, int wtype, int epi, int M, int K, bool have
     static constexpr double kFill[2][4] = {{1.3, 3.4, 3.8, 4.4}, {1.5, 5.0, 7.0, 8.0}};
     static constexpr double kBlock[2][4] = {{1.17, 1.17, 1.5, 1.78}, {2.1, 2.15, 2.4, 2.9}};
     const int cus = num_cus(), nb = K / 256;
-    QPlan best{4, 1, 1};
+    const bool two = epi == EPI_SWIGLU;
+    int from = 1, to = have_ws ? std::min(16, nb) : 1;
+    if (two && have_ws) from = to = quant_plan(job, wtype, EPI_STORE, M, K, have_ws).S;
+    QPlan best{1, two ? 2 : 1, from};
     double least = 1e30;
-    for (int fn = epi == EPI_SWIGLU ? 2 : 1; fn <= 2; ++fn) {
+    for (int fn = two ? 2 : 1; fn <= 2; ++fn) {
         // 96 rows at most with Q6_K at 256 columns: its raw blocks take the LDS
         const int fm_max = wtype == BX_TYPE_Q6_K && fn == 2 ? 3 : 4;
         for (int fm = 1; fm <= fm_max; ++fm) {
             int64_t tiles = 0;
-            const int bn = epi == EPI_SWIGLU ? 128 : 128 * fn;
+            const int bn = two ? 128 : 128 * fn;
             for (int i = 0; i < job.members; ++i) tiles += (job.N[i] + bn - 1) / bn;
             tiles *= (M + 32 * fm - 1) / (32 * fm);
-            for (int S = 1; S <= 16 && S <= nb; ++S) {
-                if (S > 1 && (!have_ws || tiles * S > cus || tiles > kSplGroups ||
+            for (int S = from; S <= to; ++S) {
+                // more slices than fill the CUs only where they are given.  The
+                // partials then fit as 32-row tiles at the latest: of the plain
+                // launch, at most cus tiles of 128 x 256, SwiGLU's are twice
+                if (S > 1 && ((tiles * S > cus && from < to) || tiles > kSplGroups ||
                               tiles * S * fm * fn * 4096 > kSplFloats))
                     break;
                 const int64_t wgs = tiles * S;
                 double block = kBlock[fn - 1][fm - 1] * (wtype == BX_TYPE_Q6_K ? 1.35 : 1.0);
                 if (wgs > cus * 7 / 8) block *= 1.0 + 0.06 * fm * fn;
-                const double t = (double)((wgs + cus - 1) / cus) * (kFill[fn - 1][fm - 1] + (nb + S - 1) / S * block) +
+                const double rounds = wgs <= cus ? 1.0 : (double)((wgs + cus - 1) / cus);
+                const double t = rounds * (kFill[fn - 1][fm - 1] + (nb + S - 1) / S * block) +
                                  (S > 1 ? 2.0 + 0.9 * fm * fn + 0.3 * S : 0.0);
                 if (t < least) {
                     least = t;

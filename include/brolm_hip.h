@@ -110,7 +110,8 @@ int bx_linear_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t
  * 256 (the MFMA GEMV of decode batches); else 0 and the caller runs the
  * unfused ops.
  * bx_linear_group_f16: n (1..3) weights of one type sharing X (q / k / v
- *   projections), Y[i] (M, N[i]) FP16, one launch.
+ *   projections), Y[i] (M, N[i]) FP16, one launch.  With quantized weights and
+ *   M >= 128 the FP32 sums may be added in another order than bx_linear_f16's.
  * bx_linear_residual_f16: H (M, N) FP32 += f16(X W^T) (o / down projection
  *   and the residual add).
  * bx_linear_swiglu_f16: Y (M, F) = f16(f16(silu(f16(X Wg^T))) * f16(X Wu^T))

@@ -147,3 +147,27 @@ def test_quant_fused_epilogues_vs_oracle(t, M, K, Ns):
            _tol(Ws[1], X, g) * _tol(Ws[2], X, u) * 1.1 + 2.0 ** -9 * np.abs(ref) + 1e-6)
     got = f16_host(act).reshape(M, Ns[1])
     assert np.all(np.abs(got - ref) <= tol), float((np.abs(got - ref) / tol).max())
+
+
+@pytest.mark.parametrize("t", QTYPES)
+@pytest.mark.parametrize("M,K,N", [(128, 2048, 2048), (128, 1024, 3072), (160, 1024, 3072), (300, 2048, 1024), (511, 4096, 130),
+                                   (200, 1280, 258), (150, 6144, 300), (129, 768, 98), (140, 14336, 64)])
+def test_quant_residual_and_swiglu_have_the_bits_of_the_separate_ops(t, M, K, N):
+    """Both add an output's K slices in the order of the plain launch, whatever
+    tiles they take."""
+    print(f"[quant fused bits] t={t} M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(M + K)
+    ws = [carrier(t, sb.random_blocks(rng, t, N * K // sb.QK[t])[0], N, K) for _ in range(2)]
+    x = f16_dev(rng.standard_normal((M, K)) * 0.02)
+    sep = [torch().empty(M * N, dtype=torch().int16, device="cuda") for _ in range(3)]
+    for w, y in zip(ws, sep):
+        call("bx_linear_f16", t, ptr(w), None, ptr(x), ptr(y), M, N, K, *lws(), stream())
+    assert np.isfinite(f16_host(sep[0])).all()
+    H0 = rng.standard_normal((M, N)).astype(np.float32)
+    H = dev(H0)
+    call("bx_linear_residual_f16", t, ptr(ws[0]), ptr(x), ptr(H), M, N, K, *lws(), stream())
+    assert np.array_equal(host(H).reshape(M, -1), H0 + f16_host(sep[0]).reshape(M, -1))
+    call("bx_linear_swiglu_f16", t, ptr(ws[0]), ptr(ws[1]), ptr(x), ptr(sep[2]), M, N, K, *lws(), stream())
+    call("bx_silu_f16", ptr(sep[0]), ptr(sep[0]), M * N, stream())
+    call("bx_mul_f16", ptr(sep[0]), ptr(sep[1]), M * N, stream())
+    assert np.array_equal(host(sep[2]), host(sep[0]))

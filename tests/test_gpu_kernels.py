@@ -170,7 +170,8 @@ def _weights(rng, t, N, K):
 def test_fused_prefill_linears_equal_unfused_ops(t, M, K, Ns):
     """bx_linear_group / _residual / _swiglu give bit-identical results to the
     separate linear, add_inplace, silu and mul launches they replace (same
-    MFMA arithmetic, same FP16 roundings): the tile GEMM at M >= 128, the MFMA
+    MFMA arithmetic, same FP16 roundings): the tile GEMM at M >= 128 (two blocks
+    of K, so one slice; a quantized group's own K slices may differ), the MFMA
     GEMV of decode batches at 3 <= M <= 16 (partial row tiles; K = 6144 in two
     row chunks of staged activations); other M decline."""
     print(f"[fused] t={t} M={M} K={K} N={Ns}", flush=True)
