@@ -19,7 +19,8 @@
 // They serve what the LDS-DMA kernels leave: quantized weights with K a
 // multiple of 256 run gemm_quant.hip (Q6_K with an even count of blocks), FP16
 // weights with K a multiple of 64 gemm_f16.hip, at any M above 16 with 16-byte
-// aligned operands (gemm_quant_ok, gemm_f16_ok).
+// aligned operands (gemm_quant_ok, gemm_f16_ok), but for FP16 shapes of few 64x64
+// tiles and short K (gemm_f16_tiles).
 #include "carrier_layout.h"
 #include "gemm_job.h"
 
@@ -504,6 +505,14 @@ int gemm_tiles_typed(int wtype, const TileJob& job, const uint16_t* bias, const 
 }
 
 }  // namespace
+
+int gemm_f16_small(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st) {
+    switch (epi) {
+        case EPI_RESID: return launch_tiles<BX_TYPE_F16, 64, 64, 4, EPI_RESID>(job, bias, X, M, K, st);
+        case EPI_SWIGLU: return launch_tiles<BX_TYPE_F16, 64, 64, 4, EPI_SWIGLU>(job, bias, X, M, K, st);
+        default: return launch_tiles<BX_TYPE_F16, 64, 64, 4, EPI_STORE>(job, bias, X, M, K, st);
+    }
+}
 
 bool gemm_tiles_ok(int M, int K);
 bool gemm_quant_ok(int wtype, const TileJob& job, const uint16_t* X, int M, int K);

@@ -19,7 +19,8 @@
 // does not; the launcher estimates the time of each shape.
 //
 // The epilogue stages the FP16 tile in LDS and stores 16 bytes a thread, rows
-// of whole lines.
+// of whole lines; at any alignment, so odd column counts take the same stores
+// (one by one they made SwiGLU 700 x 1500 x 768 16.1 us, 10.9 with them).
 #include <algorithm>
 
 #include "gemm_job.h"
@@ -29,6 +30,9 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
+typedef u4v __attribute__((aligned(2))) any16;   // eight FP16 values at any address
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef f4v __attribute__((aligned(4))) any_f4;
 
 template <int BM_, int WM_, int WN_, int NB_>
 struct FShape {
@@ -179,7 +183,6 @@ __global__ __launch_bounds__(Sh::NT, 1) void gemm_f16_kernel(TileJob job, const 
     constexpr int kChunks = BN / 8;
     const int cn = two ? kChunks / 2 : kChunks;   // chunks of output columns
     uint16_t* const Y = two ? job.Y[0] : job.Y[mem];
-    const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(epi == EPI_RESID ? (void*)job.H : (void*)Y) & 15) == 0;
     for (int i = threadIdx.x; i < BM * cn; i += Sh::NT) {
         const int row = i / cn, m = m0 + row, n = n0 + (i % cn) * 8;
         if (m >= M || n >= N) continue;
@@ -201,24 +204,26 @@ __global__ __launch_bounds__(Sh::NT, 1) void gemm_f16_kernel(TileJob job, const 
         const int64_t at = (int64_t)m * N + n;
         if (epi == EPI_RESID) {
             float* const h = job.H + at;
-            if (vec) {
-                typedef float f4 __attribute__((ext_vector_type(4)));
-                f4* const h4 = reinterpret_cast<f4*>(h);
-                f4 a = h4[0], b = h4[1];
+            if (n + 8 <= N) {
+                f4v a = *reinterpret_cast<any_f4*>(h), b = *reinterpret_cast<any_f4*>(h + 4);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     a[k] += h2f(o.h[k]);
                     b[k] += h2f(o.h[4 + k]);
                 }
-                h4[0] = a;
-                h4[1] = b;
+                *reinterpret_cast<any_f4*>(h) = a;
+                *reinterpret_cast<any_f4*>(h + 4) = b;
             } else {
-                for (int k = 0; k < 8 && n + k < N; ++k) h[k] += h2f(o.h[k]);
+#pragma unroll
+                for (int k = 0; k < 7; ++k)
+                    if (n + k < N) h[k] += h2f(o.h[k]);
             }
-        } else if (vec) {
-            *reinterpret_cast<u4v*>(Y + at) = o.v;
+        } else if (n + 8 <= N) {
+            *reinterpret_cast<any16*>(Y + at) = o.v;
         } else {
-            for (int k = 0; k < 8 && n + k < N; ++k) Y[at + k] = o.h[k];
+#pragma unroll
+            for (int k = 0; k < 7; ++k)
+                if (n + k < N) Y[at + k] = o.h[k];
         }
     }
 }
@@ -267,6 +272,15 @@ bool gemm_f16_ok(const TileJob& job, const uint16_t* X, int M, int K) {
 // x 4096: 256 x 256 1116, 256 x 128 1033, 128 x 128 1001 [815]; 2000 x 4096 x
 // 2048: 256 x 128 856, 256 x 256 699 [744]; 2000 x 2048 x 6144: 128 x 128 869,
 // 256 x 128 718 [649]; 777 x 2048 x 6144: 128 x 64 560, 128 x 128 444 [379].
+//
+// From 128 rows on and K up to 1024, up to two 64 x 64 tiles a CU also have the
+// register-staged tiles of gemm.hip, four wavefronts each (the same bits: one
+// 32x32x16 MFMA order over K): a shorter fill and epilogue, slower stages.  In us,
+// those against the best shape here: 200 x 1000 x 768 6.9 / 7.8, 300 x 2048 x 1024
+// 8.4 / 8.9, SwiGLU 300 x 3072 x 1024 11.2 / 12.8; 200 x 1024 x 2048 12.8 / 12.6, 511
+// x 512 x 4096 35.0 / 20.4.
+int gemm_f16_small(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st);
+
 int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st) {
     struct Plan {
         int bm, bn, per_cu;
@@ -292,6 +306,16 @@ int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint
         if (t < least) {
             least = t;
             best = &p;
+        }
+    }
+    if (M >= 128 && K <= 1024) {
+        const int cn = epi == EPI_SWIGLU ? 32 : 64;
+        int64_t tiles = 0;
+        for (int i = 0; i < job.members; ++i) tiles += (job.N[i] + cn - 1) / cn;
+        tiles *= (M + 63) / 64;
+        if (tiles <= 2 * (int64_t)num_cus()) {
+            const double t = 3.4 + (K / 64) * (tiles <= num_cus() ? 0.305 : 0.47);
+            if (t < least) return gemm_f16_small(epi, job, bias, X, M, K, st);
         }
     }
     return best->run(job, bias, X, M, K, epi, st);
