@@ -25,7 +25,7 @@
 // epilogue and the exchange of partials.  Measured against the tile kernels of
 // gemm.hip that ran these shapes before (one launch, weights from HBM):
 // 75 x 6144 x 2048 Q4_K 44.2 -> 13.6 us, 300 x 2048 x 6144 Q6_K 98 -> 25.3 us,
-// 2000 x 6144 x 2048 Q4_K 94 -> 79 us, SwiGLU 130 x 3000 x 1024 Q4_K 15.5 -> 13.0.
+// 2000 x 6144 x 2048 Q4_K 94 -> 79 us, SwiGLU 128 x 3072 x 1024 Q4_K 14.1 -> 7.9.
 //
 // Where the tiles leave CUs idle, S workgroups share a tile's K: each writes
 // its FP32 partials by device-scope stores to the linear workspace, the last
@@ -262,15 +262,19 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_quant_kernel(QuantJob job, c
     const int tile = tn * job.t.tiles_m + tm;
     int mem = 0;
     while (tn >= job.t.tiles_n[mem]) tn -= job.t.tiles_n[mem++];
-    const bool two = epi == EPI_SWIGLU;   // column group g of a wavefront: gate, up
+    // SwiGLU tiles: gate in the first half of the columns, up in the second (FN 2:
+    // column groups 0 and 1 of a wavefront, FN 1: wavefronts 0, 1 and 2, 3)
+    const bool two = epi == EPI_SWIGLU;
     const int N = job.t.N[mem];
     const int m0 = tm * BM, n0 = tn * (two ? BN / 2 : BN);
     const int nb = K / 256;
     const int b0 = s * nb / S, nblk = (s + 1) * nb / S - b0;   // >= 1
     const int nh = 2 * nblk;
     // first column of this wavefront in group g
-    auto col0 = [&](int g) { return n0 + 32 * wave + (two ? 0 : 128 * g); };
-    auto weight = [&](int g) { return static_cast<const unsigned char*>(two ? job.t.W[g] : job.t.W[mem]); };
+    auto col0 = [&](int g) { return n0 + (two ? 32 * (FN == 2 ? wave : wave & 1) : 32 * wave + 128 * g); };
+    auto weight = [&](int g) {
+        return static_cast<const unsigned char*>(two ? job.t.W[FN == 2 ? g : wave >> 1] : job.t.W[mem]);
+    };
 
     const uint32_t lbase = lds_addr(smem);
     unsigned char* const raw = smem + NA * Sh::kSlot + wave * Sh::kWave;
@@ -521,21 +525,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_quant_kernel(QuantJob job, c
     // ---- epilogue: a thread takes four columns of a row
     const bool vec = (N & 3) == 0;   // rows start 8 (16) bytes aligned with their base
     if (two) {
-        if constexpr (FN == 2) {
-            uint16_t* const Y = job.t.Y[0];
-            for (int i = threadIdx.x; i < BM * 32; i += kThreads) {
-                const int m = m0 + i / 32, n = n0 + (i % 32) * 4;
-                if (m >= M || n >= N) continue;
-                const unsigned char* row = smem + (i / 32) * Sh::kRow + (i % 32) * 16;
-                const f4v a = *reinterpret_cast<const f4v*>(row), b = *reinterpret_cast<const f4v*>(row + 512);
-                uint16_t o[4];
+        uint16_t* const Y = job.t.Y[0];
+        constexpr int kH = kQ / 2;   // quads of gate columns
+        for (int i = threadIdx.x; i < BM * kH; i += kThreads) {
+            const int m = m0 + i / kH, n = n0 + (i % kH) * 4;
+            if (m >= M || n >= N) continue;
+            const unsigned char* row = smem + (i / kH) * Sh::kRow + (i % kH) * 16;
+            const f4v a = *reinterpret_cast<const f4v*>(row), b = *reinterpret_cast<const f4v*>(row + kH * 16);
+            uint16_t o[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float act = h2f(f2h(silu_f32(h2f(f2h(a[k])))));
-                    o[k] = f2h(act * h2f(f2h(b[k])));
-                }
-                store4(Y + (int64_t)m * N + n, o, vec, N - n);
+            for (int k = 0; k < 4; ++k) {
+                const float act = h2f(f2h(silu_f32(h2f(f2h(a[k])))));
+                o[k] = f2h(act * h2f(f2h(b[k])));
             }
+            store4(Y + (int64_t)m * N + n, o, vec, N - n);
         }
         return;
     }
@@ -563,17 +566,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_quant_kernel(QuantJob job, c
 // epilogue plus a time per 256-element block of K (decode-bound up to FM = 2,
 // then MFMA-bound), more when every CU streams; a split adds the exchange of
 // its partials.  Example: 75 x 6144 x 2048 Q4_K takes 13.1 us as 32-row tiles,
-// 14.7 us as 96-row tiles in 4 slices, 28 us as 96 x 256 tiles.
+// 14.7 us as 96-row tiles in 4 slices, 28 us as 96 x 256 tiles.  SwiGLU has tiles
+// of 64 + 64 columns too (FN 1), for matrices whose 128 + 128 leave CUs idle: 128 x
+// 3072 x 1024 Q8_0 12.5 -> 8.6 us (10.3 on the tiles of gemm.hip), 128 x 6144 x 2048
+// 21.1 -> 15.7.
 //
 // The slices decide the order in which an output's sums are added.  A residual
 // launch has those of the plain launch, being planned alike, and SwiGLU takes
 // those of the plain launch of gate or up: both give the bits of the separate
-// ops.  (Its own slices would be faster only for Q6_K of few columns: 128 x 3072
-// x 1024 13.8 us, 15.1 so.)  q / k / v in one launch have slices of their own:
-// those of the separate launches, which fill the chip three times over, cost up
-// to twice the time (200 rows of 2048 + 1024 + 1024 columns, K = 2048, Q4_K 12.9
-// us against 28.8), so a group's sums may differ from the plain launches' in the
-// last bits of FP32.
+// ops.  q / k / v in one launch have slices of their own: those of the separate
+// launches, which fill the chip three times over, cost up to twice the time (200
+// rows of 2048 + 1024 + 1024 columns, K = 2048, Q4_K 12.9 us against 28.8), so a
+// group's sums may differ from the plain launches' in the last bits of FP32.
 struct QPlan {
     int fm, fn, S;
 };
@@ -585,14 +589,14 @@ QPlan quant_plan(const TileJob& job, int wtype, int epi, int M, int K, bool have
     const bool two = epi == EPI_SWIGLU;
     int from = 1, to = have_ws ? std::min(16, nb) : 1;
     if (two && have_ws) from = to = quant_plan(job, wtype, EPI_STORE, M, K, have_ws).S;
-    QPlan best{1, two ? 2 : 1, from};
+    QPlan best{1, 1, from};
     double least = 1e30;
-    for (int fn = two ? 2 : 1; fn <= 2; ++fn) {
+    for (int fn = 1; fn <= 2; ++fn) {
         // 96 rows at most with Q6_K at 256 columns: its raw blocks take the LDS
         const int fm_max = wtype == BX_TYPE_Q6_K && fn == 2 ? 3 : 4;
         for (int fm = 1; fm <= fm_max; ++fm) {
             int64_t tiles = 0;
-            const int bn = two ? 128 : 128 * fn;
+            const int bn = two ? 64 * fn : 128 * fn;
             for (int i = 0; i < job.members; ++i) tiles += (job.N[i] + bn - 1) / bn;
             tiles *= (M + 32 * fm - 1) / (32 * fm);
             for (int S = from; S <= to; ++S) {
@@ -606,8 +610,9 @@ QPlan quant_plan(const TileJob& job, int wtype, int epi, int M, int K, bool have
                 double block = kBlock[fn - 1][fm - 1] * (wtype == BX_TYPE_Q6_K ? 1.35 : 1.0);
                 if (wgs > cus * 7 / 8) block *= 1.0 + 0.06 * fm * fn;
                 const double rounds = wgs <= cus ? 1.0 : (double)((wgs + cus - 1) / cus);
-                const double t = rounds * (kFill[fn - 1][fm - 1] + (nb + S - 1) / S * block) +
+                double t = rounds * (kFill[fn - 1][fm - 1] + (nb + S - 1) / S * block) +
                                  (S > 1 ? 2.0 + 0.9 * fm * fn + 0.3 * S : 0.0);
+                if (two && fn == 1) t *= 1.05;   // a tie goes to the tiles that read X half as often
                 if (t < least) {
                     least = t;
                     best = QPlan{fm, fn, S};
