@@ -111,6 +111,7 @@ HIP_SYMBOLS = {
     "bx_argmax_f16": (C.c_int, [vp, i64, vp, vp, vp]),
     "bx_argmax_f16_noalloc": (C.c_int, [vp, i64, vp, vp]),
     "bx_linear_tiles_ok": (C.c_int, [C.c_int, C.c_int]),
+    "bx_linear_plan": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "bx_linear_workspace_bytes": (C.c_size_t, []),
     "bx_linear_workspace_init": (C.c_int, [vp, C.c_size_t, vp]),
     "bx_attention_varlen_f16": (C.c_int, [vp, vp, vp, C.c_int, vp, vp, C.c_int, C.c_int, C.c_int, C.c_int, vp, vp,

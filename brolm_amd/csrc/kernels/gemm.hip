@@ -520,6 +520,8 @@ int gemm_quant(int wtype, int epi, const TileJob& job, const uint16_t* bias, con
                size_t wsb, hipStream_t st);
 bool gemm_f16_ok(const TileJob& job, const uint16_t* X, int M, int K);
 int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st);
+void gemm_quant_shape(int wtype, int epi, const TileJob& job, int M, int K, bool have_ws, int* shape);
+bool gemm_f16_shape(int epi, const TileJob& job, int M, int K, int* shape);
 
 int gemm_f16(int wtype, const void* W, const uint16_t* bias, const uint16_t* X, uint16_t* Y, int M, int N, int K,
              void* ws, size_t wsb, hipStream_t st) {
@@ -585,3 +587,25 @@ int gemm_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X
 }
 
 }  // namespace bx
+
+extern "C" int bx_linear_plan(int wtype, int form, int n, const int* N, int M, int K, int have_ws, int* plan) {
+    using namespace bx;
+    if (!N || !plan || n < 1 || n > 3 || M <= 0 || K <= 0 || form < 0 || form > 2)
+        return fail(BX_EINVAL, "linear_plan: bad arguments");
+    TileJob job{};
+    job.members = n;
+    for (int i = 0; i < n; ++i) {
+        if (N[i] <= 0) return fail(BX_EINVAL, "linear_plan: bad arguments");
+        job.N[i] = N[i];
+    }
+    plan[0] = plan[1] = plan[2] = plan[3] = 0;
+    if (M <= 16) return BX_OK;
+    plan[0] = 1;
+    if (gemm_quant_ok(wtype, job, nullptr, M, K)) {
+        plan[0] = 3;
+        gemm_quant_shape(wtype, form, job, M, K, have_ws != 0, plan + 1);
+    } else if (wtype == BX_TYPE_F16 && gemm_f16_ok(job, nullptr, M, K) && gemm_f16_shape(form, job, M, K, plan + 1)) {
+        plan[0] = 2;
+    }
+    return BX_OK;
+}

@@ -255,6 +255,8 @@ using Q64 = FShape<64, 2, 1, 6>;     // 64 x 64, 2 wavefronts
 
 }  // namespace
 
+int gemm_f16_small(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st);
+
 // K in whole stages, operands aligned for 16-byte copies.
 bool gemm_f16_ok(const TileJob& job, const uint16_t* X, int M, int K) {
     if (M <= 16 || K % 64 != 0 || (reinterpret_cast<uintptr_t>(X) & 15)) return false;
@@ -279,14 +281,16 @@ bool gemm_f16_ok(const TileJob& job, const uint16_t* X, int M, int K) {
 // those against the best shape here: 200 x 1000 x 768 6.9 / 7.8, 300 x 2048 x 1024
 // 8.4 / 8.9, SwiGLU 300 x 3072 x 1024 11.2 / 12.8; 200 x 1024 x 2048 12.8 / 12.6, 511
 // x 512 x 4096 35.0 / 20.4.
-int gemm_f16_small(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st);
+namespace {
 
-int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st) {
-    struct Plan {
-        int bm, bn, per_cu;
-        double fill, idle, full;   // us a stage with few CUs at work, with all
-        int (*run)(TileJob, const uint16_t*, const uint16_t*, int, int, int, hipStream_t);
-    };
+struct Plan {
+    int bm, bn, per_cu;
+    double fill, idle, full;   // us a stage with few CUs at work, with all
+    int (*run)(TileJob, const uint16_t*, const uint16_t*, int, int, int, hipStream_t);
+};
+
+// Null: the tiles of gemm.hip.
+const Plan* f16_plan(int epi, const TileJob& job, int M, int K) {
     static const Plan kPlans[] = {
         {256, 256, 1, 12.0, 1.00, 1.65, launch<T256>}, {256, 128, 1, 9.0, 0.58, 0.92, launch<T128>},
         {128, 128, 1, 7.5, 0.37, 0.51, launch<S128>},  {128, 128, 2, 8.0, 0.57, 0.97, launch<S128x2>},
@@ -315,10 +319,24 @@ int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint
         tiles *= (M + 63) / 64;
         if (tiles <= 2 * (int64_t)num_cus()) {
             const double t = 3.4 + (K / 64) * (tiles <= num_cus() ? 0.305 : 0.47);
-            if (t < least) return gemm_f16_small(epi, job, bias, X, M, K, st);
+            if (t < least) return nullptr;
         }
     }
-    return best->run(job, bias, X, M, K, epi, st);
+    return best;
+}
+
+}  // namespace
+
+int gemm_f16_tiles(int epi, const TileJob& job, const uint16_t* bias, const uint16_t* X, int M, int K, hipStream_t st) {
+    const Plan* p = f16_plan(epi, job, M, K);
+    return p ? p->run(job, bias, X, M, K, epi, st) : gemm_f16_small(epi, job, bias, X, M, K, st);
+}
+
+// {rows, columns, workgroups per CU} of a launch's tiles; false: those of gemm.hip
+bool gemm_f16_shape(int epi, const TileJob& job, int M, int K, int* shape) {
+    const Plan* p = f16_plan(epi, job, M, K);
+    if (p) shape[0] = p->bm, shape[1] = p->bn, shape[2] = p->per_cu;
+    return p != nullptr;
 }
 
 }  // namespace bx

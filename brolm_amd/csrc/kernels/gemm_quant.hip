@@ -678,6 +678,14 @@ bool gemm_quant_ok(int wtype, const TileJob& job, const uint16_t* X, int M, int 
     return true;
 }
 
+// {rows, columns, K slices} of a launch's tiles
+void gemm_quant_shape(int wtype, int epi, const TileJob& job, int M, int K, bool have_ws, int* shape) {
+    const QPlan p = quant_plan(job, wtype, epi, M, K, have_ws);
+    shape[0] = 32 * p.fm;
+    shape[1] = 128 * p.fn;
+    shape[2] = p.S;
+}
+
 int gemm_quant(int wtype, int epi, const TileJob& t, const uint16_t* bias, const uint16_t* X, int M, int K, void* ws,
                size_t wsb, hipStream_t st) {
     const bool have_ws = ws != nullptr && wsb >= kSplCntBytes + (size_t)kSplFloats * 4;

@@ -123,6 +123,12 @@ int bx_linear_residual_f16(int wtype, const void* W, const uint16_t* X, float* H
                            size_t ws_bytes, void* stream);
 int bx_linear_swiglu_f16(int wtype, const void* Wg, const void* Wu, const uint16_t* X, uint16_t* Y, int M, int F,
                          int K, void* ws, size_t ws_bytes, void* stream);
+/* Debug: what a launch of these forms (0 plain or group, 1 residual, 2 SwiGLU with
+ * N[0] = F) runs on 16-byte aligned operands.  plan[0]: 0 the GEMVs, 1 the tiles
+ * of gemm.hip, 2 gemm_f16.hip, 3 gemm_quant.hip; plan[1..3], for 2 and 3: rows and
+ * columns of a tile, then workgroups per CU (2) or K slices (3).  No device is
+ * needed (256 CUs are assumed without one). */
+int bx_linear_plan(int wtype, int form, int n, const int* N, int M, int K, int have_ws, int* plan);
 /* Decode batches (3 <= M <= 16, K % 256 == 0) with the residual RMSNorm
  * (rms_norm_forward, dense_decoder.cpp:559, :540-550) carried between
  * launches instead of run on its own: bx_linear_residual_ss_f16 is

@@ -1,5 +1,6 @@
-"""Linears on FP16 weights at 17 rows and more (gemm_f16.hip): every tile shape
-at its edges, the epilogues, and operands it leaves to the general kernels."""
+"""Linears on FP16 weights at 17 rows and more (gemm_f16.hip): the epilogues at
+partial tiles, and operands and shapes it leaves to the general kernels.
+test_gpu_linear_tiles.py has every tile shape."""
 from __future__ import annotations
 
 import ctypes as C
@@ -32,8 +33,8 @@ def _ref(X, W):
     return X.astype(np.float64) @ W.astype(np.float64).T
 
 
-# the shapes the launcher gives to 64 x 64, 128 x 64, 128 x 128 (one and two
-# workgroups per CU), 256 x 128 and 256 x 256 tiles, with partial tiles
+# on 256 CUs: 64 x 64 tiles of gemm_f16.hip and (from 128 rows, K to 1024) of
+# gemm.hip, 128 x 128 (one and two workgroups per CU) and 256 x 256, partial tiles
 SHAPES = [(17, 1, 64), (63, 65, 128), (65, 130, 192), (129, 2049, 64), (385, 4100, 640), (700, 4097, 448),
           (2049, 1025, 512), (1100, 9000, 320), (1281, 12295, 256)]
 

@@ -1,6 +1,7 @@
-"""Linears on quantized weights at 17 rows and more (gemm_quant.hip): tile
-edges in rows and columns, K slices, the fused epilogues, and the shapes it
-leaves to the general tile kernel, against the oracle."""
+"""Linears on quantized weights at 17 rows and more (gemm_quant.hip): edges of the
+32-row tiles, K slices, the fused epilogues, and the shapes it leaves to the
+general tile kernel, against the oracle.  test_gpu_linear_tiles.py has the other
+tiles."""
 from __future__ import annotations
 
 import ctypes as C
