@@ -191,7 +191,10 @@ int bx_kv_append_f16(const uint16_t* k, const uint16_t* v, int L, int cols, int 
  * (dense_decoder.cpp:606-607; Gemma form src/gemma2.cpp:365-367).
  * q (L, n_q*hd) FP16, caches (cap, n_kv*hd) FP16, out (L, n_q*hd) FP16.
  * Row r attends keys [max(0, p-window+1), p] with p = valid_len - L + r.
- * workspace: bx_attention_workspace_bytes(L, n_q, hd, valid_len) bytes. */
+ * workspace: bx_attention_workspace_bytes(L, n_q, hd, valid_len) bytes, scratch
+ * of this call: it is written at any L (16 rows and more over long caches share
+ * their keys out over workgroups), so calls that may run at the same time (other
+ * streams, other threads) take distinct ones. */
 size_t bx_attention_workspace_bytes(int L, int n_q, int hd, int valid_len);
 int bx_attention_decode_f16(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len,
                             int n_q, int n_kv, int hd, float softcap, int window, uint16_t* out,
@@ -201,7 +204,8 @@ int bx_attention_decode_f16(const uint16_t* q, const uint16_t* Kc, const uint16_
  * (dense_decoder.cpp:737-745, the encoder's attention): q (L, n_q*hd), K / V
  * (n_keys, n_kv*hd) FP16, out (L, n_q*hd) FP16.  causal = 0: every row
  * attends all n_keys keys; causal = 1: row r attends keys [0, n_keys - L + r].
- * workspace: bx_attention_workspace_bytes(L, n_q, hd, n_keys) bytes. */
+ * workspace: bx_attention_workspace_bytes(L, n_q, hd, n_keys) bytes, used as by
+ * bx_attention_decode_f16. */
 int bx_attention_gqa_f16(const uint16_t* q, const uint16_t* K, const uint16_t* V, int L, int n_keys, int n_q,
                          int n_kv, int hd, int causal, uint16_t* out, void* workspace, void* stream);
 
@@ -210,7 +214,7 @@ int bx_attention_gqa_f16(const uint16_t* q, const uint16_t* K, const uint16_t* V
  * the newest token of its own sequence, whose rlen = lens_dev[r] keys sit in
  * cache rows base_rows_dev[r] .. + rlen - 1 (the last one its own); max_len >=
  * every rlen sizes the split.  workspace: bx_attention_workspace_bytes(rows,
- * n_q, hd, max_len) bytes. */
+ * n_q, hd, max_len) bytes, not shared by calls that may run at the same time. */
 int bx_attention_varlen_f16(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int rows,
                             const int32_t* lens_dev, const int64_t* base_rows_dev, int max_len, int n_q, int n_kv,
                             int hd, uint16_t* out, void* workspace, void* stream);

@@ -70,3 +70,37 @@ def test_attention_rows(L, keys, n_q, n_kv, hd, causal, offset):
     # is the result; scores and sums are FP32 (below 1e-5 here)
     tol = 2.0 ** -11 * (np.abs(host[2]).max() + np.abs(want)) + 1e-5
     assert (np.abs(got - want) <= tol).all(), float((np.abs(got - want) / tol).max())
+
+
+def test_attention_two_streams_with_their_own_workspaces():
+    """Calls on two streams at once, keys shared out over workgroups (records in the
+    workspace): each gives the bits it gives alone."""
+    import torch
+    from brolm_amd import _native as nat
+    hip = nat.hip()
+    L, keys, n_q, n_kv, hd, reps = 40, 2040, 16, 8, 128, 6
+    rng = np.random.default_rng(5)
+    nb = int(hip.bx_attention_workspace_bytes(L, n_q, hd, keys))
+    ops = [[torch.from_numpy(rng.standard_normal((r, n * hd)).astype(np.float16)).cuda()
+            for r, n in ((L, n_q), (keys, n_kv), (keys, n_kv))] for _ in range(2)]
+    wss = [torch.empty(nb, dtype=torch.uint8, device="cuda") for _ in range(2)]
+
+    def run(i, out, stream):
+        p = [C.c_void_p(t.data_ptr()) for t in (*ops[i], out, wss[i])]
+        assert hip.bx_attention_decode_f16(*p[:3], L, keys, n_q, n_kv, hd, C.c_float(0.0), 0, p[3], p[4],
+                                           C.c_void_p(stream.cuda_stream)) == 0, nat.hip_error()
+
+    outs = [[torch.zeros(L, n_q * hd, dtype=torch.float16, device="cuda") for _ in range(reps)] for _ in range(2)]
+    alone = [torch.zeros(L, n_q * hd, dtype=torch.float16, device="cuda") for _ in range(2)]
+    for i in range(2):
+        run(i, alone[i], torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for r in range(reps):
+        for i in range(2):
+            run(i, outs[i][r], streams[i])
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert float(alone[i].float().abs().max()) > 0
+        for r in range(reps):
+            assert torch.equal(outs[i][r], alone[i]), (i, r)
