@@ -11,7 +11,6 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -180,7 +179,7 @@ void d2h_f16_as_f32(float* dst, const void* src, std::size_t n) {
         for (int p = 1; p < parts; ++p) {
             try {
                 helpers[p] = std::thread([&, p] { err[p] = convert(p); });
-            } catch (const std::system_error&) {   // no thread to be had: this one converts
+            } catch (...) {   // no thread, or no memory for one: this thread converts
                 err[p] = convert(p);
             }
         }
