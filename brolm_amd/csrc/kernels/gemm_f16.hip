@@ -12,11 +12,12 @@
 // so the copies of the stage NB ahead go into it, and the next stage's first
 // fragments are read under the last step's MFMAs.
 //
-// What bounds it: 256 x 256 tiles read 192 KB of LDS a stage (8 wavefronts of
-// 128 x 64) and write 64 KB, 2048 cycles at 128 bytes a cycle, as long as the
-// stage's MFMAs; the clock falls to 1.6 GHz under this load.  128 x 128 tiles
-// need 1.5 times their MFMA time in LDS, but fill the chip where 256 x 256
-// does not; the launcher estimates the time of each shape.
+// What bounds it: the matrix cores, busy for 73 % of the cycles at 256 x 256 tiles
+// (SwiGLU 2048 x 12288 x 4096), at a clock that falls to 1.6 GHz under this load;
+// the LDS is active for 29 % (192 KB of fragments a stage), a third of the wave
+// cycles wait.  128 x 128 tiles read 1.5 times as much LDS for the same MFMAs, but
+// fill the chip where 256 x 256 does not; the launcher estimates the time of each
+// shape.
 //
 // The epilogue stages the FP16 tile in LDS and stores 16 bytes a thread, rows
 // of whole lines; at any alignment, so odd column counts take the same stores
