@@ -33,9 +33,9 @@
 // through registers and V transposed on its way into LDS: 2048 causal rows of
 // 32 / 8 heads of 128 100 -> 51.7 us (660 TFLOP/s), 500 rows bidirectional
 // of 16 heads 17.8 -> 9.3 us, 700 rows after 2000 of 16 heads 87 -> 36 us,
-// 64 rows after 2000 of 16 heads 62 -> 12.1 us.  Calls of up to 64 rows over 33
-// to 64 keys are the exception (64 rows of 16 heads 5.1 -> 5.6 us): a fragment
-// of 32 rows has twice the serial work of one of 16.
+// 64 rows after 2000 of 16 heads 62 -> 12.1 us.  Up to 128 keys are one tile and
+// have a kernel of their own (fa_one_tile_kernel): a fragment of 32 rows has
+// twice the serial work of one of 16, and a merge costs 0.5 to 0.9 us.
 #include <algorithm>
 
 #include "attention_core.h"
@@ -56,8 +56,7 @@ template <int HD, int KS, int NK>
 struct FaShape {
     static constexpr int TK = KS == 4 ? 128 : 64;       // keys per tile
     static constexpr int WK = TK / KS;                  // keys per wavefront and tile
-    static constexpr int SK = 32 * NK;                  // keys per step: NK fragments of 32
-    static_assert(WK == SK || WK == 2 * SK);
+    static_assert(WK == 32 * NK);                       // NK fragments of 32 keys
     static constexpr int RB = HD * 2;                   // bytes per key row
     static constexpr int CH = HD / 8;                   // 16-byte chunks per key row
     static constexpr int RPC = 1024 / RB;               // rows per copy instruction
@@ -204,9 +203,8 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
         if (kb + 1 < kb_end) issue(kb + 1, cur ^ 1);
         const unsigned char* const kt = smem + cur * S::kBuf;
         const unsigned char* const vt = kt + S::kTile;
-        auto step = [&](int st) {   // keys st .. st + SK - 1 of the wavefront's share
-            const int key0 = kb * S::TK + kw * S::WK + st;
-            if (key0 > any_see) return;
+        const int key0 = kb * S::TK + kw * S::WK;
+        if (key0 <= any_see) {
             // fragments of 32 keys some query sees
             const bool more = NK > 1 && key0 + 32 <= any_see;
             // S^T: lane l, register r of s[t] holds key 32 t + 8 (r / 4) + 4 lh + r % 4
@@ -223,7 +221,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
                 fa_h8 kf[HD / 16];
 #pragma unroll
                 for (int d = 0; d < HD / 16; ++d)
-                    kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + (st + 32 * t) * S::RB + (((2 * d) ^ kx) << 4));
+                    kf[d] = *reinterpret_cast<const fa_h8*>(kt + ka + t * 32 * S::RB + (((2 * d) ^ kx) << 4));
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int d = 0; d < HD / 16; ++d)
@@ -239,7 +237,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
 #pragma unroll
                     for (int j = 0; j < ND; ++j) {
                         const int c = 4 * j + vcol;
-                        const int k1 = st + 32 * t + 16 * u + vkey, k2 = k1 + 8;
+                        const int k1 = 32 * t + 16 * u + vkey, k2 = k1 + 8;
                         const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + vb8;
                         const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + vb8;
                         const fa_h4 lo = __builtin_bit_cast(
@@ -251,7 +249,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
             };
             values(0);
             __builtin_amdgcn_sched_barrier(0);
-            if (key0 + S::SK - 1 > all_see) {
+            if (key0 + S::WK - 1 > all_see) {
 #pragma unroll
                 for (int t = 0; t < NK; ++t)
 #pragma unroll
@@ -270,8 +268,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
             // well inside FP16).  A query that has seen no key yet has m =
             // -inf: its first visible tile moves it, and until then every
             // weight is exp2(-inf - finite) = 0 (nm below).
-            // (Two steps of one tile: any larger max, as one step would have it.)
-            if (__any(mx > m + (S::WK > S::SK ? 0.f : 8.f))) {
+            if (__any(mx > m + 8.f)) {
                 const float mnew = fmaxf(m, mx);
                 const float alpha = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);
                 l *= alpha;
@@ -299,9 +296,7 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
                     for (int j = 0; j < ND; ++j)
                         o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u][j], pb[u], o[j], 0, 0, 0);
             }
-        };
-        step(0);
-        if constexpr (S::WK > S::SK) step(S::SK);
+        }
         if (kb + 1 < kb_end) land(cur ^ 1);
         tile_wait();
     }
@@ -401,6 +396,152 @@ __global__ __launch_bounds__(kFaThreads, !AL && KS == 4 ? 1 : 2) void fa_kernel(
     }
 }
 
+// One tile of up to 64 or 128 keys (the smallest calls): fragments of 16 rows, whose
+// chain of S, softmax and P V is half as long as that of 32, on
+// v_mfma_f32_16x16x32_f16.  A workgroup has 64 rows of one head, a wavefront 16 of
+// them; K and V come by LDS-DMA (through registers where they are not on 16 bytes),
+// requested with q, and are waited for once.  (K straight into the operands, by
+// every wavefront, took 64 KB through the L1 of a CU: 5.4 us for 64 rows and keys.)
+// What bounds it: the launch and that one memory round trip.  16 rows and keys of 16
+// heads of 128 3.1 us, 64 rows and keys 4.0, 128 rows and keys 4.9; fa_kernel 4.8, 5.9
+// and 6.5, the 16-row fragments with K and V staged through registers 4.1, 5.1 and 6.9.
+constexpr int kOneTile = 128;
+
+template <int HD, int NT, bool AL>
+__global__ __launch_bounds__(kFaThreads, 2) void fa_one_tile_kernel(const uint16_t* __restrict__ q,
+                                                                   const uint16_t* __restrict__ Kc,
+                                                                   const uint16_t* __restrict__ Vc, int L, int valid_len,
+                                                                   int n_q, int n_kv, int bidir,
+                                                                   uint16_t* __restrict__ out) {
+    using S = FaShape<HD, 1, 2>;   // the layout of a key row
+    constexpr int ND = HD / 16, kTile = 16 * NT * S::RB, P = 16 * NT / S::RPC / 4;
+    __shared__ __align__(1024) unsigned char tiles[2 * kTile];   // K, then V
+    const unsigned char* const vt = tiles + kTile;
+    const int rt = (int)blockIdx.x, head = (int)blockIdx.y, g = head / (n_q / n_kv);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lq = lane & 15, lg = lane >> 4;
+    const int64_t qstride = (int64_t)n_q * HD, kvstride = (int64_t)n_kv * HD;
+    const int row0 = 64 * rt + 16 * wave, row = row0 + lq, p0 = valid_len - L;
+    const int last_key = bidir ? valid_len - 1 : min(p0 + row, valid_len - 1);
+    const int any_see = bidir ? valid_len - 1 : min(p0 + row0 + 15, valid_len - 1);
+
+    // q rows: B operand, lane l holds query l % 16, d 32 s + 8 (l / 16) ..
+    fa_h8 qf[HD / 32];
+    {
+        const uint16_t* const qrow = q + (int64_t)min(row, L - 1) * qstride + (int64_t)head * HD + 8 * lg;
+#pragma unroll
+        for (int d = 0; d < HD / 32; ++d)
+            qf[d] = __builtin_bit_cast(fa_h8, (u4v)*reinterpret_cast<const fa_any16*>(qrow + 32 * d));
+    }
+    // wavefront w copies rows RPC (w P + j) .. of the tile; keys past the end repeat
+    // the last one
+    const unsigned char* const kb0 = reinterpret_cast<const unsigned char*>(Kc + (int64_t)g * HD);
+    const unsigned char* const vb0 = reinterpret_cast<const unsigned char*>(Vc + (int64_t)g * HD);
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(tiles) + wave * P * 1024);
+    u4v reg[AL ? 1 : 2 * P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int r = S::RPC * (wave * P + j) + lane / S::CH;
+        const uint32_t off = (uint32_t)min(r, valid_len - 1) * (uint32_t)(kvstride * 2) +
+                             (uint32_t)(((lane % S::CH) ^ S::swz(r)) * 16);
+        if constexpr (AL) {
+            dma16(off, kb0, dst + j * 1024);
+            dma16(off, vb0, dst + kTile + j * 1024);
+        } else {
+            reg[2 * j] = *reinterpret_cast<const fa_any16*>(kb0 + off);
+            reg[2 * j + 1] = *reinterpret_cast<const fa_any16*>(vb0 + off);
+        }
+    }
+    if constexpr (!AL) {
+#pragma unroll
+        for (int j = 0; j < 2 * P; ++j)
+            *reinterpret_cast<u4v*>(tiles + (j & 1) * kTile + (wave * P + j / 2) * 1024 + lane * 16) = reg[j];
+    }
+    wait_vm_barrier<0>();
+    if (row0 >= L) return;
+
+    // S^T: lane l, register r of s[t] holds key 16 t + 4 (l / 16) + r of query l % 16
+    fa_f4 s[NT];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        s[t] = fa_f4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        if (16 * t <= any_see) {
+            s[t] = fa_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int d = 0; d < HD / 32; ++d) {
+                const int k = 16 * t + lq;   // A operand: lane l holds key l % 16, the same d
+                const fa_h8 kf = *reinterpret_cast<const fa_h8*>(tiles + k * S::RB + (((4 * d + lg) ^ S::swz(k)) << 4));
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[d], s[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (16 * t + 4 * lg + r > last_key) s[t][r] = -INFINITY;
+                mx = fmaxf(mx, s[t][r]);
+            }
+        }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    const float sl2 = 1.4426950408889634f / sqrtf((float)HD);
+    const float m = fmaxf(mx, __shfl_xor(mx, 32)) * sl2, nm = m == -INFINITY ? 0.f : -m;
+    float l = 0.f;
+    fa_h8 pb[NT / 2];   // B operands of 32 keys: 16 of one fragment and 16 of the next
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float p = __builtin_amdgcn_exp2f(fmaf(s[t][r], sl2, nm));
+            l += p;
+            pb[t / 2][4 * (t % 2) + r] = (_Float16)p;
+        }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // O^T: d = 16 j + 4 (l / 16) + r of query l % 16
+    const int tkey = 4 * lg + (lq >> 2), tcol = (lq & 3) >> 1, tb = (lq & 1) * 8;
+    fa_f4 o[ND];
+#pragma unroll
+    for (int j = 0; j < ND; ++j) o[j] = fa_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < NT / 2; ++u) {
+        if (32 * u > any_see) break;
+#pragma unroll
+        for (int j = 0; j < ND; ++j) {
+            const int c = 2 * j + tcol, k1 = 32 * u + tkey, k2 = k1 + 16;
+            const unsigned char* const a1 = vt + k1 * S::RB + ((c ^ S::swz(k1)) << 4) + tb;
+            const unsigned char* const a2 = vt + k2 * S::RB + ((c ^ S::swz(k2)) << 4) + tb;
+            const fa_h4 lo = __builtin_bit_cast(
+                fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a1));
+            const fa_h4 hi = __builtin_bit_cast(
+                fa_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_s4*)a2));
+            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pb[u],
+                                                          o[j], 0, 0, 0);
+        }
+    }
+    if (row >= L) return;
+    const float inv = 1.0f / l;
+    uint16_t* const orow = out + (int64_t)row * qstride + (int64_t)head * HD + 4 * lg;
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+        u2v w;
+        w.x = (uint32_t)f2h(o[j][0] * inv) | ((uint32_t)f2h(o[j][1] * inv) << 16);
+        w.y = (uint32_t)f2h(o[j][2] * inv) | ((uint32_t)f2h(o[j][3] * inv) << 16);
+        *reinterpret_cast<fa_any8*>(orow + 16 * j) = w;
+    }
+}
+
+template <int HD, bool AL>
+int fa_one_tile_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q,
+                       int n_kv, int bidir, uint16_t* out, hipStream_t st) {
+    if (n_q > 65535) return fail(BX_EINVAL, "attention: too many heads");
+    const dim3 grid((unsigned)((L + 63) / 64), (unsigned)n_q);
+    if (valid_len <= 64)
+        fa_one_tile_kernel<HD, 4, AL><<<grid, kFaThreads, 0, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out);
+    else
+        fa_one_tile_kernel<HD, 8, AL><<<grid, kFaThreads, 0, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out);
+    return launch_check("attention (one tile)");
+}
+
 template <int HD, int KS, int NK, bool AL>
 int fa_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q, int n_kv,
               int bidir, int gb, int sp, float* recs, uint16_t* out, hipStream_t st) {
@@ -437,10 +578,11 @@ int fa_dispatch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L
     const int G = n_q / n_kv, cus = num_cus();
     const int64_t frags = (int64_t)((L + 31) / 32) * n_q;
     float* const recs = static_cast<float*>(ws);
-    // the smallest calls: one tile, no merge (16 heads of 128: 16 rows and keys
-    // 4.1 us, KS 2 4.8; 64 rows and keys 5.6, KS 2 5.9)
-    if (valid_len <= 64)
-        return fa_launch<HD, 1, 1, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, 1, 1, recs, out, st);
+    // 128 keys in 64 KB: two workgroups a CU, more rounds of them cost more than
+    // 32-row fragments (2048 rows of 32 heads 14.6 us against 14.0; of 16 heads 7.9
+    // against 10.2)
+    if (valid_len <= 64 || (valid_len <= kOneTile && (int64_t)((L + 63) / 64) * n_q <= 2 * cus))
+        return fa_one_tile_launch<HD, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
     if (frags <= cus && valid_len > 256) {
         const int tiles = (valid_len + 127) / 128, room = attn_ws_splits(L, valid_len);
         int sp = (int)std::min<int64_t>({cus / frags, room, tiles / 2});

@@ -24,10 +24,12 @@ def _exact(q, K, V, n_q, n_kv, hd, causal):
 
 @pytest.mark.parametrize("offset", [0, 1])   # 1: operands 2 bytes off the 16-byte grid
 @pytest.mark.parametrize("L,keys,n_q,n_kv,hd,causal", [
-    # one tile of keys, in one step or two
+    # one tile of keys in 16-row fragments: 64 keys, then 128, wavefronts without a row
     (16, 16, 4, 4, 64, 1), (31, 33, 4, 2, 128, 1), (33, 64, 6, 2, 128, 0), (64, 64, 16, 2, 128, 1), (17, 32, 2, 1, 64, 1),
+    (300, 47, 6, 3, 64, 0), (16, 65, 4, 2, 128, 1), (32, 100, 7, 7, 64, 1), (128, 128, 4, 1, 128, 1), (65, 127, 3, 1, 64, 0),
+    (113, 113, 2, 2, 64, 1), (50, 97, 5, 5, 128, 0),
     # keys of a tile over two wavefronts: one row to a few tiles, wavefronts without a row
-    (16, 65, 4, 2, 128, 1), (32, 100, 7, 7, 64, 1), (64, 256, 8, 1, 64, 0),
+    (16, 130, 4, 2, 128, 1), (64, 256, 8, 1, 64, 0),
     (129, 129, 7, 1, 128, 1), (700, 701, 16, 2, 128, 1), (600, 1, 16, 2, 64, 0),
     # over four, and then over workgroups too
     (300, 300, 8, 2, 128, 1), (257, 257, 8, 8, 64, 0), (17, 1500, 8, 2, 128, 1), (65, 1023, 4, 4, 64, 1),
