@@ -533,7 +533,6 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_one_tile_kernel(const uint16
 template <int HD, bool AL>
 int fa_one_tile_launch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L, int valid_len, int n_q,
                        int n_kv, int bidir, uint16_t* out, hipStream_t st) {
-    if (n_q > 65535) return fail(BX_EINVAL, "attention: too many heads");
     const dim3 grid((unsigned)((L + 63) / 64), (unsigned)n_q);
     if (valid_len <= 64)
         fa_one_tile_kernel<HD, 4, AL><<<grid, kFaThreads, 0, st>>>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out);
@@ -581,7 +580,8 @@ int fa_dispatch(const uint16_t* q, const uint16_t* Kc, const uint16_t* Vc, int L
     // 128 keys in 64 KB: two workgroups a CU, more rounds of them cost more than
     // 32-row fragments (2048 rows of 32 heads 14.6 us against 14.0; of 16 heads 7.9
     // against 10.2)
-    if (valid_len <= 64 || (valid_len <= kOneTile && (int64_t)((L + 63) / 64) * n_q <= 2 * cus))
+    if (n_q <= 65535 &&
+        (valid_len <= 64 || (valid_len <= kOneTile && (int64_t)((L + 63) / 64) * n_q <= 2 * cus)))
         return fa_one_tile_launch<HD, AL>(q, Kc, Vc, L, valid_len, n_q, n_kv, bidir, out, st);
     if (frags <= cus && valid_len > 256) {
         const int tiles = (valid_len + 127) / 128, room = attn_ws_splits(L, valid_len);
